@@ -251,6 +251,41 @@ struct SplitLayerIn {
 hipError_t launch_decode_split(int count, const SplitLayerIn *in, const SplitPlan *plans,
                                int64_t M, int x_bf16, unsigned *tickets, hipStream_t st);
 
+// ---- k_slim.hip ----
+// The forward for few tokens: up to kMaxSlimSegs layers with the same batch
+// in one pair of launches (launch_slim_prep, then launch_slim).  Layers with
+// the same xp share their X.  The plan's tickets start at
+// kDecodeTileCounterBase; calls sharing them must be stream-ordered.
+constexpr int kMaxSlimSegs = 4;
+struct SlimPlan {
+  bool ok = false;
+  int G = 0, P = 0, R = 0, chunks = 0;
+  uint32_t lds = 0;
+  int S[kMaxSlimSegs] = {}, groups[kMaxSlimSegs] = {}, nz[kMaxSlimSegs] = {};
+  size_t part_floats[kMaxSlimSegs] = {};  // scratch of the K slices' sums
+  size_t xp_bytes[kMaxSlimSegs] = {};     // scratch of the X planes
+};
+struct SlimIn {
+  DevQW w;
+  const void *x;   // M x K
+  const float *a;  // r x K
+  int64_t r;       // 0: no adapter
+  const float *lb; // N x r
+  float s;
+  float *t1p;      // nz x M x r partial T1s, written by the preparation (r > 0)
+  float *t1;       // M x r, their sum (or nullptr)
+  float *y;        // M x N
+  int beta;        // 1: y += the result
+  void *xp;        // plan.xp_bytes (16-byte aligned)
+  float *part;     // plan.part_floats
+};
+bool slim_ok(const DevQW &w, const void *x, int x_bf16, const float *a, int64_t M, int64_t r);
+SlimPlan slim_plan(int count, const DevQW *w, const int64_t *r, int64_t M, int x_bf16);
+hipError_t launch_slim_prep(int count, const SlimIn *in, const SlimPlan &p, int64_t M,
+                            int x_bf16, hipStream_t st);
+hipError_t launch_slim(int count, const SlimIn *in, const SlimPlan &p, int64_t M,
+                       unsigned *tickets, hipStream_t st);
+
 // ---- k_elem.hip ----
 hipError_t launch_axpy_inplace(float *y, const float *x, int64_t n,
                                hipStream_t s);  // y += x

@@ -74,6 +74,19 @@ struct DevBuf {
     cap = want;
     return p;
   }
+  // False, with the buffer empty, when the device has no such block left.
+  bool try_ensure(size_t bytes) {
+    if (bytes <= cap) return true;
+    release();
+    const size_t want = (bytes + 255) / 256 * 256;
+    if (hipMalloc(&p, want) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+      return false;
+    }
+    cap = want;
+    return true;
+  }
   void release() {
     if (p) (void)hipFree(p);
     p = nullptr;
@@ -94,6 +107,23 @@ struct Carve {
     return t;
   }
   std::vector<char *> bind(DevBuf &b) { return bind_at((char *)b.ensure(total())); }
+  // Binds to `b` unless that needs memory that cannot be had now: a larger
+  // buffer during a stream capture (an allocation would end the capture), or
+  // more than the device has left.  For paths with a fallback that needs
+  // less.
+  bool try_bind(DevBuf &b, hipStream_t s, std::vector<char *> *out) {
+    const size_t need = total();
+    if (need > b.cap) {
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+      }
+      if (!b.try_ensure(need)) return false;
+    }
+    *out = bind_at((char *)b.p);
+    return true;
+  }
   std::vector<char *> bind_at(char *base) {
     std::vector<char *> out;
     for (size_t s : sizes) {
@@ -503,6 +533,53 @@ static bool forward_accumulates(const DevQW &W, const qh_lora *l, const void *x,
   return qh::nf4_fast_ok(W) && qh::bf16_gemm_ok(W, x, K, K);
 }
 
+// ---- the forward for few tokens (k_slim.hip) ------------------------------
+bool takes_slim(const DevQW &W, const qh_lora *l, const void *x, int xdt, int64_t M) {
+  return qh::slim_ok(W, x, xdt == QH_BF16, l ? l->a : nullptr, M, l ? (int64_t)l->r : 0);
+}
+
+// `count` layers, each on its own x (layers with the same x share its
+// preparation); with `beta` y += the result.  False, with nothing launched,
+// where its scratch cannot be had (see Carve::try_bind) or no plan covers the
+// group: the caller runs the layers on the paths with smaller scratch.
+bool slim_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora *const *l,
+              const void *const *x, int xdt, int64_t M, float *const *y, float *const *t1_out,
+              int beta, hipStream_t s) {
+  if (count > (size_t)qh::kMaxSlimSegs) return false;
+  const int xb = xdt == QH_BF16, n = (int)count;
+  int64_t rs[qh::kMaxSlimSegs] = {};
+  for (int i = 0; i < n; ++i) rs[i] = l[i] ? (int64_t)l[i]->r : 0;
+  const qh::SlimPlan pl = qh::slim_plan(n, W, rs, M, xb);
+  if (!pl.ok) return false;
+  Carve c;
+  size_t it[qh::kMaxSlimSegs], ix[qh::kMaxSlimSegs], ip[qh::kMaxSlimSegs];
+  int own[qh::kMaxSlimSegs];
+  for (int i = 0; i < n; ++i) {
+    own[i] = i;
+    for (int j = 0; j < i && own[i] == i; ++j)
+      if (x[j] == x[i] && W[j].cols == W[i].cols) own[i] = own[j];
+    it[i] = c.add((size_t)pl.nz[i] * M * rs[i] * 4);
+    ix[i] = c.add(own[i] == i ? pl.xp_bytes[i] : 0);
+    ip[i] = c.add(pl.part_floats[i] * 4);
+  }
+  std::vector<char *> p;
+  if (!c.try_bind(ctx->scratch, s, &p)) return false;
+  qh::SlimIn in[qh::kMaxSlimSegs] = {};
+  for (int i = 0; i < n; ++i) {
+    in[i].w = W[i], in[i].x = x[i], in[i].y = y[i], in[i].beta = beta;
+    in[i].xp = p[ix[own[i]]], in[i].part = (float *)p[ip[i]];
+    if (l[i]) {
+      in[i].a = l[i]->a, in[i].lb = l[i]->b, in[i].r = rs[i];
+      in[i].s = l[i]->alpha / (float)l[i]->r;  // lora.rs:64-66
+      in[i].t1p = (float *)p[it[i]];
+      in[i].t1 = t1_out ? t1_out[i] : nullptr;
+    }
+  }
+  timed(ctx, "slim_prep", s, [&] { return qh::launch_slim_prep(n, in, pl, M, xb, s); });
+  timed(ctx, "forward_slim", s, [&] { return qh::launch_slim(n, in, pl, M, ctx->tickets, s); });
+  return true;
+}
+
 // ---- fused forward on device pointers -----------------------------------
 // With `accumulate` y += the result; only the bf16-MFMA path (the one
 // forward_accumulates names) does that, every other path refuses it before
@@ -529,6 +606,9 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
     if (lora && t1_out) t1_dev(ctx, x, xe, M, K, l, t1_out, s);
     return;
   }
+  if (takes_slim(W, l, x, xdt, M) &&
+      slim_dev(ctx, 1, &W, &l, &x, xdt, M, &y, &t1_out, accumulate ? 1 : 0, s))
+    return;
   const bool fast = qh::nf4_fast_ok(W);
   // Small batches: the MFMA decode kernels (batch <= 16, K % 256 == 0), else
   // the VALU GEMV (batch <= 4, K % 64 == 0); both need 16-byte aligned rows
@@ -898,6 +978,12 @@ void forward_shared_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora
                         const void *x, int xdt, size_t batch, float *const *y,
                         float *const *t1_out, hipStream_t s) {
   const int64_t M = (int64_t)batch, K = W[0].cols;
+  bool slim = count <= (size_t)qh::kMaxSlimSegs;
+  for (size_t i = 0; i < count && slim; ++i) slim = takes_slim(W[i], l[i], x, xdt, M);
+  if (slim) {
+    const void *const xs[qh::kMaxSlimSegs] = {x, x, x, x};
+    if (slim_dev(ctx, count, W, l, xs, xdt, M, y, t1_out, 0, s)) return;
+  }
   if (!shared_ok(count, W, l, x, nullptr, M)) {
     for (size_t i = 0; i < count; ++i)
       forward_dev(ctx, W[i], l[i], x, xdt, batch, y[i], t1_out ? t1_out[i] : nullptr, s);
