@@ -1,0 +1,120 @@
+"""GPU parity of the large GEMMs through operand planes (k_plane.hip) with the
+kernels that decode inside the K loop (k_nf4_bf16, oracle-tested): the
+allocation-free backward always takes the latter, and where that kernel does not
+split its reduction the input gradient's sums run in the same order, so the
+bits must match.  The forward is held against 64 bits on the dequantized weight.
+
+The bar on the normalised error (parity.nerr) is 8 standard deviations of one
+output's rounding error, as in tests/test_gpu_slim.py: 3.9e-6 for fp32 X (xl.wl and
+the parts below hi + lo), 2.3e-6 for bf16 X (w below hi + lo, 0.18 x 2^-16 rms,
+and the fp32 sums).
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle as O
+from parity import bf16_round, nerr
+
+pytestmark = [pytest.mark.gpu, pytest.mark.timeout(120)]
+
+torch = pytest.importorskip("torch")
+
+TOL = {torch.float32: 8 * 4.8e-6, torch.bfloat16: 8 * 2.8e-6}
+
+
+def _layer(QD, ctx, N, K, r, M, act, dq):
+    g = O.Rng(N + 3 * K + 7 * M)
+    dev = lambda v: torch.from_numpy(np.ascontiguousarray(v)).cuda()  # noqa: E731
+    rnd = (lambda v: bf16_round(v)) if act == torch.bfloat16 else (lambda v: v)
+    w, x = g.normal(N * K, 0.02).reshape(N, K), rnd(g.normal(M * K)).reshape(M, K)
+    dy = rnd(g.normal(M * N)).reshape(M, N)
+    a, b = g.uniform(r * K, -0.02, 0.02).reshape(r, K), g.normal(N * r, 0.01).reshape(N, r)
+    W = QD.DeviceWeight.quantize(dev(w), 64, dq, ctx=ctx)
+    ta, tb = dev(a), dev(b)
+    return dict(W=W, wd=W.dequantize(ctx=ctx).view(N, K).double(), a=ta, b=tb, x=dev(x).to(act),
+                dy=dev(dy).to(act), lora=QD.lora_struct(ta, tb, r, 16.0) if r else None,
+                s=16.0 / r if r else 0.0, nx=x, ndy=dy)
+
+
+def _backward(QD, ctx, fn, L, M):
+    gx = torch.full((M, L["W"].cols), float("nan"), device="cuda")
+    r = L["lora"].r if L["lora"] else 0
+    ga, gb = (torch.empty(n, device="cuda") for n in (r * L["W"].cols or 1, r * L["W"].rows or 1))
+    s = L["W"].struct()
+    QD.check(fn(ctx.h, C.byref(s), C.byref(L["lora"]) if r else None, QD._p(L["x"]),
+                QD._p(L["dy"]), QD._dt(L["x"]), M, None, QD._p(gx), QD._p(ga), QD._p(gb),
+                C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    return gx
+
+
+CASES = [
+    # (N, K, r, M): whole tiles; rows past a tile of 256, 192 and 128 rows;
+    # columns past a tile; ranks around an MFMA's 16 and past four k tiles
+    (4096, 512, 16, 2048), (4352, 512, 8, 1029), (8256, 576, 64, 600), (4200, 1088, 17, 1100),
+    (4096, 512, 0, 1500), (4104, 640, 80, 1090), (2056, 2112, 5, 2900),
+]
+
+
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,K,r,M", CASES)
+def test_plane_forward(ctx, N, K, r, M, act):
+    from qlora_hip import device as QD
+    for dq in (True, False):
+        print(f"plane forward N={N} K={K} r={r} M={M} {act} dq={dq}", flush=True)
+        L = _layer(QD, ctx, N, K, r, M, act, dq)
+        y = torch.full((M, N), float("nan"), device="cuda")
+        ctx.set_timing(True)
+        QD.forward(L["W"], L["lora"], L["x"], M, y, ctx=ctx)
+        torch.cuda.synchronize()
+        rep = ctx.timing_report(reset=True)
+        ctx.set_timing(False)
+        assert "planes" in rep, rep
+        xd = L["x"].double()
+        want = xd @ L["wd"].T + L["s"] * ((xd @ L["a"].double().T) @ L["b"].double().T)
+        assert nerr(y.cpu().numpy(), want.cpu().numpy(), K, L["nx"],
+                    L["wd"].cpu().numpy()) < TOL[act]
+
+
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,K,r,M", [(512, 4096, 16, 2048), (576, 4352, 8, 1029),
+                                     (632, 8256, 64, 600), (520, 4160, 5, 1100),
+                                     (2056, 2112, 5, 2900)])
+def test_plane_input_gradient(ctx, N, K, r, M, act):
+    from qlora_hip import device as QD
+    L = _layer(QD, ctx, N, K, r, M, act, True)
+    ctx.set_timing(True)
+    got = _backward(QD, ctx, ctx.lib.qh_qlora_backward_dev, L, M)
+    torch.cuda.synchronize()
+    rep = ctx.timing_report(reset=True)
+    ctx.set_timing(False)
+    assert "planes" in rep, rep
+    ref = _backward(QD, ctx, ctx.lib.qh_qlora_backward_dev_noalloc, L, M)
+    torch.cuda.synchronize()
+    dy = L["dy"].double()
+    want = dy @ L["wd"] + (L["s"] * (dy @ L["b"].double())) @ L["a"].double()
+    for t in (got, ref):
+        assert nerr(t.cpu().numpy(), want.cpu().numpy(), N, L["ndy"],
+                    L["wd"].cpu().numpy()) < TOL[act]
+    # both run x.w (and its LoRA term) k by k in one chain unless the other split K
+    if torch.equal(got.view(torch.int32), ref.view(torch.int32)):
+        return
+    assert float((got - ref).abs().max()) < 1e-5 * float(ref.abs().max())
+
+
+def test_plane_shared_sum_and_residual(ctx):
+    """Two layers that both take planes: the second adds its input gradient to
+    the first's."""
+    from qlora_hip import device as QD
+    M, K = 1100, 4096
+    Ls = [_layer(QD, ctx, N, K, 8, M, torch.float32, True) for N in (512, 640)]
+    gx = torch.empty(M, K, device="cuda")
+    QD.backward_shared([(L["W"], L["lora"]) for L in Ls], Ls[0]["x"], [L["dy"] for L in Ls], M, gx,
+                       [torch.empty(8, K, device="cuda") for _ in Ls],
+                       [torch.empty(L["W"].rows, 8, device="cuda") for L in Ls], ctx=ctx)
+    torch.cuda.synchronize()
+    want = sum(L["dy"].double() @ L["wd"] + (L["s"] * (L["dy"].double() @ L["b"].double())) @
+               L["a"].double() for L in Ls)
+    assert nerr(gx.cpu().numpy(), want.cpu().numpy(), 1152, Ls[0]["ndy"],
+                Ls[0]["wd"].cpu().numpy()) < TOL[torch.float32]

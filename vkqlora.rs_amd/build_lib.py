@@ -25,7 +25,7 @@ ARCH = "gfx950"
 SOURCES = ["runtime.cpp", "nf4_file.cpp", "k_quant.hip", "k_gemm.hip", "k_gemm_bf16.hip",
            "k_gemv.hip",
            "k_dstream.hip", "k_dsplit.hip", "k_adam.hip", "k_elem.hip",
-           "k_block.hip", "k_rank.hip", "k_slim.hip"]
+           "k_block.hip", "k_rank.hip", "k_slim.hip", "k_plane.hip"]
 
 COMMON = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17",

@@ -251,6 +251,38 @@ struct SplitLayerIn {
 hipError_t launch_decode_split(int count, const SplitLayerIn *in, const SplitPlan *plans,
                                int64_t M, int x_bf16, unsigned *tickets, hipStream_t st);
 
+// ---- k_plane.hip: large GEMMs through bf16 operand planes ----
+// An operand (rows x K) as planes: fp32 p[r * ld + k] (PLANE_ROWK) or
+// p[k * ld + r] (PLANE_KROW), times scale, as hi and lo parts; bf16
+// p[r * ld + k] as one part; NF4 weight rows (r = W row) or columns (r = W
+// column, K = W rows; rows % 64 == 0) as hi and lo parts.
+enum PlaneForm { PLANE_ROWK, PLANE_KROW, PLANE_NF4_ROW, PLANE_NF4_COL };
+struct PlaneSrc {
+  int form, bf16;
+  const void *p;
+  int64_t ld, rows, K;
+  float scale;
+  DevQW w;
+  void *dst;
+};
+// Whether an M x N output over K goes through planes.
+bool plane_ok(int64_t M, int64_t N, int64_t K);
+// Bytes of an A operand's (M rows) and a B operand's (N rows) planes.
+size_t plane_a_bytes(int64_t M, int64_t K, int parts);
+size_t plane_b_bytes(int64_t N, int64_t K);
+hipError_t launch_planes(const PlaneSrc *src, int count, hipStream_t st);  // count <= 4
+// C (M x N) = A . B^T + A2 . B2^T (+ C with beta), the sums of k_gemm_bf16.hip's
+// unsplit kernels in their order.
+struct PlaneGemm {
+  const void *a, *b, *a2, *b2;
+  int a_parts;
+  int64_t M, N, K, K2;
+  float *c;
+  int64_t ldc;
+  int beta;
+};
+hipError_t launch_plane_gemm(const PlaneGemm &p, hipStream_t st);
+
 // ---- k_slim.hip ----
 // The forward for few tokens: up to kMaxSlimSegs layers with the same batch
 // in one pair of launches (launch_slim_prep, then launch_slim).  Layers with

@@ -580,6 +580,40 @@ bool slim_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora *const *l
   return true;
 }
 
+// ---- large GEMMs through operand planes (k_plane.hip) ---------------------
+// Scratch slots of one GEMM's planes (A, the weight, the LoRA term's two).
+struct PlaneSlots {
+  size_t a, b, a2, b2;
+  PlaneSlots(Carve &c, bool on, int64_t M, int64_t N, int64_t K, int64_t r, int parts)
+      : a(c.add(on ? qh::plane_a_bytes(M, K, parts) : 0)),
+        b(c.add(on ? qh::plane_b_bytes(N, K) : 0)),
+        a2(c.add(on && r ? qh::plane_a_bytes(M, r, 2) : 0)),
+        b2(c.add(on && r ? qh::plane_b_bytes(N, r) : 0)) {}
+};
+
+// C (M x N) = X . op(W)^T + P2 . (scale Q2)^T (+ C with beta): the forward
+// (w_form PLANE_NF4_ROW: X M x K, P2 = T1, Q2 = B, N x r) or the input gradient
+// (PLANE_NF4_COL: X = dY, P2 = Ds, Q2 = A^T, A r x N).
+void plane_gemm_dev(qh_ctx *ctx, const std::vector<char *> &p, const PlaneSlots &ps, const char *name,
+                    const DevQW &W, int w_form, const void *x, int a32, int64_t M, int64_t N,
+                    int64_t K, const float *p2, const float *q2, int64_t r, float scale, float *c,
+                    int beta, hipStream_t s) {
+  qh::PlaneSrc src[4] = {};
+  src[0].form = qh::PLANE_ROWK, src[0].bf16 = !a32, src[0].p = x, src[0].ld = K, src[0].rows = M;
+  src[0].K = K, src[0].scale = 1.0f, src[0].dst = p[ps.a];
+  src[1].form = w_form, src[1].w = W, src[1].rows = N, src[1].K = K, src[1].dst = p[ps.b];
+  if (r) {
+    src[2].form = qh::PLANE_ROWK, src[2].p = p2, src[2].ld = r, src[2].rows = M, src[2].K = r;
+    src[2].scale = 1.0f, src[2].dst = p[ps.a2];
+    src[3].form = w_form == qh::PLANE_NF4_ROW ? qh::PLANE_ROWK : qh::PLANE_KROW;
+    src[3].p = q2, src[3].ld = w_form == qh::PLANE_NF4_ROW ? r : N, src[3].rows = N, src[3].K = r;
+    src[3].scale = scale, src[3].dst = p[ps.b2];
+  }
+  timed(ctx, "planes", s, [&] { return qh::launch_planes(src, r ? 4 : 2, s); });
+  const qh::PlaneGemm g{p[ps.a], p[ps.b], p[ps.a2], p[ps.b2], a32 ? 2 : 1, M, N, K, r, c, N, beta};
+  timed(ctx, name, s, [&] { return qh::launch_plane_gemm(g, s); });
+}
+
 // ---- fused forward on device pointers -----------------------------------
 // With `accumulate` y += the result; only the bf16-MFMA path (the one
 // forward_accumulates names) does that, every other path refuses it before
@@ -683,11 +717,19 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
   }
   const int y_splits = bf16 ? qh::bf16_gemm_splits(M, N, K) : base_splits(M, N, K);
   Carve c;
-  size_t i_t1 = c.add(lora && !t1_out ? (size_t)M * r * 4 : 0);
-  size_t i_w32 = c.add(fast ? 0 : (size_t)W.n * 4);
-  size_t i_p1 = c.add(!lora ? 0 : t1_dense ? dt1.partial_bytes() : partial_floats(gt1) * 4);
-  size_t i_p2 = c.add(y_splits > 1 ? (size_t)y_splits * M * N * 4 : 0);
-  auto p = c.bind(ctx->scratch);
+  const size_t i_t1 = c.add(lora && !t1_out ? (size_t)M * r * 4 : 0);
+  const size_t i_w32 = c.add(fast ? 0 : (size_t)W.n * 4);
+  const size_t i_p1 =
+      c.add(!lora ? 0 : t1_dense ? dt1.partial_bytes() : partial_floats(gt1) * 4);
+  const size_t i_p2 = c.add(y_splits > 1 ? (size_t)y_splits * M * N * 4 : 0);
+  // large GEMMs through operand planes where their scratch can be had
+  bool plane = bf16 && qh::plane_ok(M, N, K);
+  Carve cp = c;
+  cp.sizes[i_p2] = 0;
+  const PlaneSlots slots(cp, plane, M, N, K, r, xe == qh::E_F32 ? 2 : 1);
+  std::vector<char *> p;
+  plane = plane && cp.try_bind(ctx->scratch, s, &p);
+  if (!plane) p = c.bind(ctx->scratch);
   float *t1 = lora ? (t1_out ? t1_out : (float *)p[i_t1]) : nullptr;
 
   if (lora && t1_rank) {
@@ -709,6 +751,11 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
     float *w32 = (float *)p[i_w32];
     timed(ctx, "dequantize", s, [&] { return qh::launch_dequantize(W, w32, s); });
     B = op(w32, K, qh::ROWK, qh::E_F32);
+  }
+  if (plane) {
+    plane_gemm_dev(ctx, p, slots, "forward_gemm_bf16", W, qh::PLANE_NF4_ROW, x, xe == qh::E_F32, M,
+                   N, K, t1, lora ? l->b : nullptr, r, sc, y, accumulate ? 1 : 0, s);
+    return;
   }
   if (bf16) {
     // bf16 MFMA against the weight's hi / lo bf16 parts (X exact when bf16,
@@ -846,13 +893,23 @@ void backward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
   size_t i_p4 = c.add(!lora ? 0 : ga_dense ? dga.partial_bytes() : partial_floats(gga) * 4);
   const bool bf16 = fast && qh::bf16_gemm_ok(W, dy, N, N);
   const int gx_splits = bf16 ? qh::bf16_gemm_splits(M, K, N) : base_splits(M, K, N);
-  size_t i_p5 = c.add(gx_splits > 1 ? (size_t)gx_splits * M * K * 4 : 0);
+  const size_t i_p5 = c.add(gx_splits > 1 ? (size_t)gx_splits * M * K * 4 : 0);
   if (plan_bytes) {
     *plan_bytes = c.total();
     return;
   }
-  ScratchSrc grow{&ctx->scratch, nullptr, 0};
-  auto p = (src ? *src : grow).bind(c);
+  // the input gradient through operand planes where its scratch can be had
+  // (never in the fixed region, whose bound is part of the interface)
+  bool plane = bf16 && !src && qh::plane_ok(M, K, N);
+  Carve cp = c;
+  cp.sizes[i_p5] = 0;
+  const PlaneSlots slots(cp, plane, M, K, N, r, a32 ? 2 : 1);
+  std::vector<char *> p;
+  plane = plane && cp.try_bind(ctx->scratch, s, &p);
+  if (!plane) {
+    ScratchSrc grow{&ctx->scratch, nullptr, 0};
+    p = (src ? *src : grow).bind(c);
+  }
 
   const float *t1 = nullptr;
   float *ds = nullptr;
@@ -913,6 +970,11 @@ void backward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
       }
     }
   }
+  if (plane) {
+    plane_gemm_dev(ctx, p, slots, "grad_x_gemm_bf16", W, qh::PLANE_NF4_COL, dy, a32, M, K, N, ds,
+                   lora ? l->a : nullptr, r, 1.0f, gx, accumulate ? 1 : 0, s);
+    return;
+  }
   if (bf16) {
     // grad_x = dY . W + Ds . A on bf16 MFMA (dY exact when bf16, split when fp32)
     qh::Bf16GemmArgs b{};
@@ -959,6 +1021,11 @@ bool shared_ok(size_t count, const DevQW *W, const qh_lora *const *l, const void
                const void *const *dy, int64_t M) {
   if (count < 2 || count > kMaxShared || count > (size_t)qh::kMaxBf16Segs) return false;
   const int64_t K = W[0].cols;
+  // members that are all large GEMMs run through operand planes one by one
+  bool planes = true;
+  for (size_t i = 0; i < count; ++i)
+    planes = planes && (dy ? qh::plane_ok(M, K, W[i].rows) : qh::plane_ok(M, W[i].rows, K));
+  if (planes) return false;
   for (size_t i = 0; i < count; ++i) {
     if (W[i].cols != K || W[i].rows == 0 || W[i].kind != W[0].kind) return false;
     if (!qh::nf4_fast_ok(W[i]) || !qh::bf16_gemm_ok(W[i], x, K, K)) return false;
