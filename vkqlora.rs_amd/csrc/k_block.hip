@@ -389,13 +389,20 @@ __global__ __launch_bounds__(kBlock) void k_swiglu_bwd(const float *gate, const 
 }
 
 // ---- softmax cross-entropy (llama.rs:487-514) ---------------------------------
-// One workgroup of 1024 threads per row.  Each thread holds up to CH float4
-// chunks of the row in registers (chunk c of thread t covers float4 index
-// c * 1024 + t; CH = 4: 16 384 logits of a row).  Pass 1: the row max; pass 2: sum of exp(v - max); pass 3:
-// dlogits = exp(v - max) / sum / seq, minus 1/seq at the target.  A row
+// One workgroup of 1024 threads per row.  The row's body, from its first 16-byte
+// boundary, is read as float4 (V4; the up to three values before it and after
+// it by one thread each).  Each thread holds up to CH chunks of the body in
+// registers (chunk c of thread t covers float4 index c * 1024 + t; CH = 4: 16 384
+// logits of a row).  Pass 1: the row max; pass 2: sum of exp(v - max); pass 3:
+// dlogits = exp(v - max) / (sum seq), minus 1/seq at the target.  A row
 // longer than the cache (STREAM) reads its remainder twice: once for a
 // running max and sum (folded into pass 1) and once to write it.  terms[row] receives
 // (logit[target] - max - ln(sum)) / seq; the loss is -sum(terms) (k_loss).
+// The quotient is one double product with the reciprocal of sum seq, rounded
+// once: two float divisions per element took more issue slots than the rest
+// (2048 rows of 128256: 588 -> 570 us; of 49152: 211 -> 183, 4.4 TB/s for one
+// read and one write).  Rows that start off 16 bytes (a vocabulary that is no
+// multiple of 4) used to be read value by value: 200 rows of 129401 148 -> 71 us.
 // dlogits may alias logits: every read of the row precedes the first
 // barrier after it, and each element is written by the thread that read it.
 template <int CH, bool V4, bool STREAM>
@@ -408,12 +415,15 @@ __global__ __launch_bounds__(kCeBlock) void k_softmax_ce(const float *logits,
   __shared__ float red[kCeBlock / 64];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t row = blockIdx.x;
-  const float *lr = logits + row * vocab;
-  float *dr = dlogits + row * vocab;
-  const int64_t nv = V4 ? (vocab >> 2) : vocab;  // vectors of E floats in the row
   const uint32_t tgt = targets[row];
   const bool tgt_ok = (int64_t)tgt < vocab;
-  const float xt = (tid == 0 && tgt_ok) ? lr[tgt] : 0.0f;
+  const float xt = (tid == 0 && tgt_ok) ? logits[row * vocab + tgt] : 0.0f;
+  // the body starts `head` elements into the row (both buffers are 16-byte
+  // aligned); thread t < 3 takes the value after it, thread 4 + t before it
+  const int head = V4 ? (int)min((int64_t)(-(row * vocab) & 3), vocab) : 0;
+  const float *lr = logits + row * vocab + head;
+  float *dr = dlogits + row * vocab + head;
+  const int64_t nv = V4 ? ((vocab - head) >> 2) : vocab;  // vectors of E floats in the body
 
   auto load = [&](int64_t c, float (&v)[E]) {
     if (V4) {
@@ -438,8 +448,10 @@ __global__ __launch_bounds__(kCeBlock) void k_softmax_ce(const float *logits,
       for (int e = 0; e < E; ++e) mx = fmaxf(mx, cache[c][e]);
     }
   }
-  const bool has_tail = V4 && tid < (vocab & 3);
-  const float tail = has_tail ? lr[(nv << 2) + tid] : 0.0f;
+  const int ntail = (int)((vocab - head) & 3);
+  const bool has_tail = V4 && (tid < ntail || (tid >= 4 && tid < 4 + head));
+  const int64_t jt = tid < 4 ? (nv << 2) + tid : tid - 4 - head;  // its place in the body
+  const float tail = has_tail ? lr[jt] : 0.0f;
   // STREAM: the part of the row past the register cache (and the tail) in
   // one online pass: running max m_s and sum s_s of exp(v - m_s)
   float m_s = -INFINITY, s_s = 0.0f;
@@ -512,9 +524,11 @@ __global__ __launch_bounds__(kCeBlock) void k_softmax_ce(const float *logits,
   sum = s[0];
 
   const float inv_seq = 1.0f / fseq;
+  const double inv = 1.0 / ((double)sum * (double)fseq);
+  const int64_t jtgt = (int64_t)tgt - head;
   auto grad = [&](float v, int64_t j) {
-    float d = expf(v - mx) / sum / fseq;
-    if (j == (int64_t)tgt) d -= inv_seq;
+    float d = (float)((double)expf(v - mx) * inv);
+    if (j == jtgt) d -= inv_seq;
     return d;
   };
 #pragma unroll
@@ -547,7 +561,7 @@ __global__ __launch_bounds__(kCeBlock) void k_softmax_ce(const float *logits,
       dr[q] = grad(v[0], q);
     }
   }
-  if (has_tail) dr[(nv << 2) + tid] = grad(tail, (nv << 2) + tid);
+  if (has_tail) dr[jt] = grad(tail, jt);
   if (tid == 0) terms[row] = tgt_ok ? (xt - mx - logf(sum)) / fseq : NAN;
 }
 
@@ -709,7 +723,7 @@ hipError_t launch_softmax_ce(const float *logits, const uint32_t *targets, int64
                              hipStream_t s) {
   if (seq > 0) {
     const float fseq = (float)seq;
-    const bool v4 = vocab % 4 == 0 && aligned16(logits) && aligned16(dlogits);
+    const bool v4 = aligned16(logits) && aligned16(dlogits);
     const int64_t nv = v4 ? vocab / 4 : vocab;
     const int64_t per = (nv + kCeBlock - 1) / kCeBlock;  // vectors per thread
     const dim3 g((unsigned)seq), b(kCeBlock);
