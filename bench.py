@@ -492,9 +492,15 @@ def prefill_bench(args, ctx, torch, dev, QD, act_dtype):
     fk = kern.get("forward_gemm_bf16") or kern.get("forward_gemm")
     if fk:
         bf = "forward_gemm_bf16" in kern
-        ach = fwd_flops / (fk["avg_ms"] * 1e9)
+        # the pass that writes the operands as bf16 planes belongs to the GEMM
+        # (the mean of the forward's and the input gradient's, alike in size)
+        gemm_ms = fk["avg_ms"] + kern.get("planes", dict(avg_ms=0.0))["avg_ms"]
+        ach = fwd_flops / (gemm_ms * 1e9)
         roof = dict(bound="mfma",
-                    kernel=("forward_gemm_bf16 (k_nf4_bf16 forward: NF4 dequant in the K loop, "
+                    kernel=("planes + forward_gemm_bf16 (k_planes: NF4 and activations to bf16 "
+                            f"planes; k_plane_gemm: {mfma_per_product} bf16 MFMAs per product)"
+                            if bf and "planes" in kern else
+                            "forward_gemm_bf16 (k_nf4_bf16 forward: NF4 dequant in the K loop, "
                             f"{mfma_per_product} bf16 MFMAs per product)" if bf
                             else "forward_gemm (k_gemm NF4 fwd, fp32 MFMA)"),
                     achieved=ach, unit="TFLOP/s", flops_per_launch=fwd_flops,

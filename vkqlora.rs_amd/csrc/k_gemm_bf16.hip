@@ -712,7 +712,10 @@ hipError_t run_bf16(const Bf16GemmArgs &g0, int splits, float *partial, hipStrea
 
 // Block shape and reduction splits by problem size.
 //  large:  256 x 256 or 256 x 128 tiles, 8 waves, for problems with at least
-//          256 tiles of 256 x 256 (MFMA-bound: C3, C5);
+//          256 tiles of 256 x 256 (MFMA-bound); such a problem comes here
+//          only where the operand planes of k_plane.hip cannot have their
+//          scratch (4096^3 in fp32 400 us here, 350 with planes), or in a
+//          group that also holds smaller layers;
 //  medium: 128 x 128 tiles, 8 waves, loads two steps ahead, two 32-wide
 //          sub-steps per barrier (one when there are more tiles than CUs,
 //          so that two blocks share a CU), for 160 or more tiles of
