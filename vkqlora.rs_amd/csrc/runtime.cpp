@@ -17,10 +17,15 @@
 #include <string>
 #include <vector>
 
+#include "dev_buf.h"
 #include "qh_internal.h"
 
+using qh::Carve;
+using qh::check;
+using qh::DevBuf;
 using qh::DevQW;
 using qh::GemmArgs;
+using qh::GpuError;
 using qh::Operand;
 
 namespace {
@@ -51,89 +56,6 @@ std::string fmt(const char *f, ...) {
   return buf;
 }
 
-struct GpuError {
-  std::string msg;
-};
-
-void check(hipError_t e, const char *what) {
-  if (e != hipSuccess) throw GpuError{std::string(what) + ": " + hipGetErrorString(e)};
-}
-
-// Growable device buffer.
-struct DevBuf {
-  void *p = nullptr;
-  size_t cap = 0;
-  void *ensure(size_t bytes) {
-    if (bytes <= cap) return p;
-    if (p) check(hipFree(p), "hipFree");
-    p = nullptr;
-    cap = 0;
-    size_t want = bytes < 256 ? 256 : bytes;
-    want = (want + 255) / 256 * 256;
-    check(hipMalloc(&p, want), "hipMalloc");
-    cap = want;
-    return p;
-  }
-  // False, with the buffer empty, when the device has no such block left.
-  bool try_ensure(size_t bytes) {
-    if (bytes <= cap) return true;
-    release();
-    const size_t want = (bytes + 255) / 256 * 256;
-    if (hipMalloc(&p, want) != hipSuccess) {
-      (void)hipGetLastError();
-      p = nullptr;
-      return false;
-    }
-    cap = want;
-    return true;
-  }
-  void release() {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    cap = 0;
-  }
-};
-
-// Bump allocator over one DevBuf: sizes are laid out first, then carved.
-struct Carve {
-  std::vector<size_t> sizes;
-  size_t add(size_t bytes) {
-    sizes.push_back((bytes + 255) / 256 * 256);
-    return sizes.size() - 1;
-  }
-  size_t total() const {
-    size_t t = 0;
-    for (size_t s : sizes) t += s;
-    return t;
-  }
-  std::vector<char *> bind(DevBuf &b) { return bind_at((char *)b.ensure(total())); }
-  // Binds to `b` unless that needs memory that cannot be had now: a larger
-  // buffer during a stream capture (an allocation would end the capture), or
-  // more than the device has left.  For paths with a fallback that needs
-  // less.
-  bool try_bind(DevBuf &b, hipStream_t s, std::vector<char *> *out) {
-    const size_t need = total();
-    if (need > b.cap) {
-      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-      if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return false;
-      }
-      if (!b.try_ensure(need)) return false;
-    }
-    *out = bind_at((char *)b.p);
-    return true;
-  }
-  std::vector<char *> bind_at(char *base) {
-    std::vector<char *> out;
-    for (size_t s : sizes) {
-      out.push_back(base);
-      base += s;
-    }
-    return out;
-  }
-};
-
 // Where a call's device scratch comes from: the context's growable buffer,
 // or a fixed region of known capacity (the allocation-free entry point,
 // whose callers have checked the size before any launch).
@@ -141,8 +63,8 @@ struct ScratchSrc {
   DevBuf *grow = nullptr;
   char *fixed = nullptr;
   size_t cap = 0;
-  std::vector<char *> bind(Carve &c) {
-    if (grow) return c.bind(*grow);
+  std::vector<char *> bind(Carve &c, hipStream_t s) {
+    if (grow) return c.bind(*grow, s);
     if (c.total() > cap) throw GpuError{"scratch larger than the fixed region"};
     return c.bind_at(fixed);
   }
@@ -167,6 +89,9 @@ struct qh_ctx {
   std::mutex mu;
   DevBuf stage[10];  // host-API staging
   DevBuf scratch;    // internal scratch of the fused paths
+  // Operand planes of the large GEMMs, two orders of magnitude above the rest:
+  // a buffer of their own, so that the scratch does not move when they grow.
+  DevBuf planes;
   DevBuf block_tmp[2];  // intermediate activations of the MLP block calls
   // Zero-initialised counters of kernels whose last workgroup finishes a
   // reduction; each such kernel leaves its counter at zero again.
@@ -479,7 +404,7 @@ void t1_dev(qh_ctx *ctx, const void *x, int xe, int64_t M, int64_t K, const qh_l
   if (dt.ok()) {
     Carve c;
     size_t ip = c.add(dt.partial_bytes());
-    auto p = c.bind(ctx->scratch);
+    auto p = c.bind(ctx->scratch, s);
     timed(ctx, "t1_gemm", s, [&] { return dt.run((float *)p[ip], s); });
     return;
   }
@@ -488,7 +413,7 @@ void t1_dev(qh_ctx *ctx, const void *x, int xe, int64_t M, int64_t K, const qh_l
   g.splits = choose_splits(M, r, K);
   Carve c;
   size_t ip = c.add(partial_floats(g) * 4);
-  auto p = c.bind(ctx->scratch);
+  auto p = c.bind(ctx->scratch, s);
   timed(ctx, "t1_gemm", s, [&] { return qh::launch_gemm(g, (float *)p[ip], s); });
 }
 
@@ -581,7 +506,7 @@ bool slim_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora *const *l
 }
 
 // ---- large GEMMs through operand planes (k_plane.hip) ---------------------
-// Scratch slots of one GEMM's planes (A, the weight, the LoRA term's two).
+// Slots of one GEMM's planes (A, the weight, the LoRA term's two).
 struct PlaneSlots {
   size_t a, b, a2, b2;
   PlaneSlots(Carve &c, bool on, int64_t M, int64_t N, int64_t K, int64_t r, int parts)
@@ -656,7 +581,7 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
     writes_y("forward_dev: y += on the GEMV path");
     Carve cg;
     size_t i_t1 = cg.add(lora && !t1_out ? (size_t)M * r * 4 : 0);
-    auto pg = cg.bind(ctx->scratch);
+    auto pg = cg.bind(ctx->scratch, s);
     float *t1 = lora ? (t1_out ? t1_out : (float *)pg[i_t1]) : nullptr;
     const int xb = xe == qh::E_BF16;
     if (lora)
@@ -687,7 +612,7 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
       Carve cs;
       size_t i_t1 = cs.add(lora && !t1_out ? (size_t)M * r * 4 : 0);
       size_t i_pt = cs.add(sp.part_floats * 4);
-      auto ps = cs.bind(ctx->scratch);
+      auto ps = cs.bind(ctx->scratch, s);
       float *t1 = lora ? (t1_out ? t1_out : (float *)ps[i_t1]) : nullptr;
       const int xb = xe == qh::E_BF16;
       if (lora)
@@ -722,14 +647,13 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
   const size_t i_p1 =
       c.add(!lora ? 0 : t1_dense ? dt1.partial_bytes() : partial_floats(gt1) * 4);
   const size_t i_p2 = c.add(y_splits > 1 ? (size_t)y_splits * M * N * 4 : 0);
-  // large GEMMs through operand planes where their scratch can be had
+  // large GEMMs through operand planes where their memory can be had
   bool plane = bf16 && qh::plane_ok(M, N, K);
-  Carve cp = c;
-  cp.sizes[i_p2] = 0;
+  Carve cp;
   const PlaneSlots slots(cp, plane, M, N, K, r, xe == qh::E_F32 ? 2 : 1);
-  std::vector<char *> p;
-  plane = plane && cp.try_bind(ctx->scratch, s, &p);
-  if (!plane) p = c.bind(ctx->scratch);
+  std::vector<char *> pp;
+  plane = plane && cp.try_bind(ctx->planes, s, &pp);
+  auto p = c.bind(ctx->scratch, s);
   float *t1 = lora ? (t1_out ? t1_out : (float *)p[i_t1]) : nullptr;
 
   if (lora && t1_rank) {
@@ -753,7 +677,7 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
     B = op(w32, K, qh::ROWK, qh::E_F32);
   }
   if (plane) {
-    plane_gemm_dev(ctx, p, slots, "forward_gemm_bf16", W, qh::PLANE_NF4_ROW, x, xe == qh::E_F32, M,
+    plane_gemm_dev(ctx, pp, slots, "forward_gemm_bf16", W, qh::PLANE_NF4_ROW, x, xe == qh::E_F32, M,
                    N, K, t1, lora ? l->b : nullptr, r, sc, y, accumulate ? 1 : 0, s);
     return;
   }
@@ -794,7 +718,7 @@ void forward_add_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *
     forward_dev(ctx, W, l, x, xdt, batch, y, t1_out, s, true);
     return;
   }
-  float *t = (float *)tmp.ensure(batch * (size_t)W.rows * 4);
+  float *t = (float *)tmp.ensure(batch * (size_t)W.rows * 4, s);
   forward_dev(ctx, W, l, x, xdt, batch, t, t1_out, s);
   timed(ctx, "residual_add", s, [&] {
     return qh::launch_axpy_inplace(y, t, (int64_t)(batch * (size_t)W.rows), s);
@@ -898,18 +822,15 @@ void backward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
     *plan_bytes = c.total();
     return;
   }
-  // the input gradient through operand planes where its scratch can be had
+  // the input gradient through operand planes where their memory can be had
   // (never in the fixed region, whose bound is part of the interface)
   bool plane = bf16 && !src && qh::plane_ok(M, K, N);
-  Carve cp = c;
-  cp.sizes[i_p5] = 0;
+  Carve cp;
   const PlaneSlots slots(cp, plane, M, K, N, r, a32 ? 2 : 1);
-  std::vector<char *> p;
-  plane = plane && cp.try_bind(ctx->scratch, s, &p);
-  if (!plane) {
-    ScratchSrc grow{&ctx->scratch, nullptr, 0};
-    p = (src ? *src : grow).bind(c);
-  }
+  std::vector<char *> pp;
+  plane = plane && cp.try_bind(ctx->planes, s, &pp);
+  ScratchSrc grow{&ctx->scratch, nullptr, 0};
+  auto p = (src ? *src : grow).bind(c, s);
 
   const float *t1 = nullptr;
   float *ds = nullptr;
@@ -971,7 +892,7 @@ void backward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
     }
   }
   if (plane) {
-    plane_gemm_dev(ctx, p, slots, "grad_x_gemm_bf16", W, qh::PLANE_NF4_COL, dy, a32, M, K, N, ds,
+    plane_gemm_dev(ctx, pp, slots, "grad_x_gemm_bf16", W, qh::PLANE_NF4_COL, dy, a32, M, K, N, ds,
                    lora ? l->a : nullptr, r, 1.0f, gx, accumulate ? 1 : 0, s);
     return;
   }
@@ -1061,7 +982,7 @@ void forward_shared_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora
   size_t it[kMaxShared];
   for (size_t i = 0; i < count; ++i)
     it[i] = c.add(l[i] && !(t1_out && t1_out[i]) ? (size_t)M * l[i]->r * 4 : 0);
-  auto p = c.bind(ctx->scratch);
+  auto p = c.bind(ctx->scratch, s);
   float *t1[kMaxShared];
   qh::RankJobs jt{};
   for (size_t i = 0; i < count; ++i) {
@@ -1109,7 +1030,7 @@ void backward_shared_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lor
                      nullptr, i > 0);
         continue;
       }
-      float *tmp = (float *)ctx->block_tmp[1].ensure((size_t)M * K * 4);
+      float *tmp = (float *)ctx->block_tmp[1].ensure((size_t)M * K * 4, s);
       backward_dev(ctx, W[i], l[i], x, dy[i], adt, batch, t1i, tmp, ga[i], gb[i], s);
       timed(ctx, "residual_add", s,
             [&] { return qh::launch_axpy_inplace(gx, tmp, (int64_t)(M * K), s); });
@@ -1129,7 +1050,7 @@ void backward_shared_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lor
     id[i] = c.add(mr);
   }
   const size_t ip = c.add(splits > 1 ? (size_t)splits * M * K * 4 : 0);
-  auto p = c.bind(ctx->scratch);
+  auto p = c.bind(ctx->scratch, s);
   const float *t1[kMaxShared];
   float *ds[kMaxShared];
   qh::RankJobs jt{}, jd{}, jg{};
@@ -1188,7 +1109,7 @@ void matmul_dev(qh_ctx *ctx, int opk, const float *a, const float *b, size_t m,
   g.splits = choose_splits(g.M, g.N, g.K);
   Carve cv;
   size_t ip = cv.add(partial_floats(g) * 4);
-  auto p = cv.bind(ctx->scratch);
+  auto p = cv.bind(ctx->scratch, s);
   timed(ctx, "matmul", s, [&] { return qh::launch_gemm(g, (float *)p[ip], s); });
 }
 
@@ -1301,6 +1222,7 @@ void qh_ctx_destroy(qh_ctx *ctx) {
   }
   for (auto &b : ctx->stage) b.release();
   ctx->scratch.release();
+  ctx->planes.release();
   for (auto &b : ctx->block_tmp) b.release();
   if (ctx->tickets) (void)hipFree(ctx->tickets);
   delete ctx;
@@ -1407,7 +1329,7 @@ qh_status qh_quantize_nf4_dev(qh_ctx *ctx, const float *d_w, size_t rows,
     hipStream_t s = pick_stream(ctx, stream);
     float *tmp = nullptr;
     if (double_quant && block_size != 64)
-      tmp = (float *)ctx->scratch.ensure(div_ceil(n, block_size) * 4 + 16);
+      tmp = (float *)ctx->scratch.ensure(div_ceil(n, block_size) * 4 + 16, s);
     timed(ctx, "quantize", s, [&] { return qh::launch_quantize(d_w, (int64_t)n, (int64_t)block_size, double_quant ? 1 : 0,
                               d_codes, d_scales, d_scale_codes, d_absmax, tmp, s); });
     return QH_OK;
@@ -1687,7 +1609,7 @@ qh_status qh_qlora_forward_group_dev(qh_ctx *ctx, size_t count, const qh_qweight
           slot[q] = c.add(d_t1s && d_t1s[i] ? 0 : (size_t)M * loras[i]->r * 4);
           pslot[q] = c.add(plan[q].ok ? plan[q].part_floats * 4 : 0);
         }
-        auto p = c.bind(ctx->scratch);
+        auto p = c.bind(ctx->scratch, s);
         std::vector<float *> t1(idx.size());
         for (size_t q = 0; q < idx.size(); ++q)
           t1[q] = d_t1s && d_t1s[idx[q]] ? d_t1s[idx[q]] : (float *)p[slot[q]];
@@ -2118,8 +2040,9 @@ static qh_status check_dev_rows(size_t rows, size_t h) {
   return QH_OK;
 }
 
-static float *dw_scratch(qh_ctx *ctx, size_t rows, size_t h) {
-  return (float *)ctx->scratch.ensure(qh::rmsnorm_dw_scratch_floats((int64_t)rows, (int)h) * 4);
+static float *dw_scratch(qh_ctx *ctx, size_t rows, size_t h, hipStream_t s) {
+  return (float *)ctx->scratch.ensure(qh::rmsnorm_dw_scratch_floats((int64_t)rows, (int)h) * 4,
+                                      s);
 }
 
 qh_status qh_rmsnorm(qh_ctx *ctx, const float *x, size_t x_len, const float *w, size_t h,
@@ -2169,7 +2092,7 @@ qh_status qh_rmsnorm_backward(qh_ctx *ctx, const float *x, size_t x_len, const f
     float *d_dw = dw ? alloc_f32(ctx, 3, h) : nullptr;
     // dx over dy only without dw: the dw stage reads dy after dx is written
     float *d_dx = dw ? alloc_f32(ctx, 4, x_len) : d_dy;
-    float *scr = dw ? dw_scratch(ctx, rows, h) : nullptr;
+    float *scr = dw ? dw_scratch(ctx, rows, h, s) : nullptr;
     timed(ctx, "rmsnorm_backward", s, [&] {
       return qh::launch_rmsnorm_bwd(d_x, d_w, d_dy, d_dx, d_dw, scr, (int64_t)rows, (int)h,
                                     eps, s);
@@ -2190,7 +2113,7 @@ qh_status qh_rmsnorm_backward_dev(qh_ctx *ctx, const float *d_x, const float *d_
     return fail(QH_ERR_INVALID_CONFIG, "dx may alias dy only when dw is not requested");
   return guarded(ctx, [&] {
     hipStream_t s = pick_stream(ctx, stream);
-    float *scr = d_dw ? dw_scratch(ctx, rows, h) : nullptr;
+    float *scr = d_dw ? dw_scratch(ctx, rows, h, s) : nullptr;
     timed(ctx, "rmsnorm_backward", s, [&] {
       return qh::launch_rmsnorm_bwd(d_x, d_w, d_dy, d_dx, d_dw, scr, (int64_t)rows, (int)h,
                                     eps, s);
@@ -2280,7 +2203,7 @@ qh_status qh_softmax_cross_entropy(qh_ctx *ctx, const float *logits, size_t logi
     uint32_t *d_t = (uint32_t *)ctx->stage[1].ensure(seq * 4 + 16);
     if (seq) check(hipMemcpyAsync(d_t, targets, seq * 4, hipMemcpyHostToDevice, s), "upload");
     float *d_loss = alloc_f32(ctx, 2, 1);
-    float *terms = (float *)ctx->scratch.ensure(seq * 4 + 16);
+    float *terms = (float *)ctx->scratch.ensure(seq * 4 + 16, s);
     timed(ctx, "softmax_cross_entropy", s, [&] {
       return qh::launch_softmax_ce(d_l, d_t, (int64_t)seq, (int64_t)vocab, d_loss, d_l, terms, s);
     });
@@ -2298,7 +2221,7 @@ qh_status qh_softmax_cross_entropy_dev(qh_ctx *ctx, const float *d_logits,
   if (st != QH_OK) return st;
   return guarded(ctx, [&] {
     hipStream_t s = pick_stream(ctx, stream);
-    float *terms = (float *)ctx->scratch.ensure(seq * 4 + 16);
+    float *terms = (float *)ctx->scratch.ensure(seq * 4 + 16, s);
     timed(ctx, "softmax_cross_entropy", s, [&] {
       return qh::launch_softmax_ce(d_logits, d_targets, (int64_t)seq, (int64_t)vocab, d_loss,
                                    d_dlogits, terms, s);
@@ -2412,7 +2335,7 @@ qh_status qh_mlp_backward_dev(qh_ctx *ctx, const qh_mlp_block *b, const qh_mlp_c
     hipStream_t s = pick_stream(ctx, stream);
     const size_t h = b->hidden, f = b->inter;
     // llama.rs:554-574 (MLP branch of block_backward)
-    float *d_act = (float *)ctx->block_tmp[0].ensure(seq * f * 4);
+    float *d_act = (float *)ctx->block_tmp[0].ensure(seq * f * 4, s);
     backward_dev(ctx, make_devqw(b->down), b->down_lora, c->act, d_dx_out, QH_F32, seq,
                  b->down_lora ? c->t1_down : nullptr, d_act,
                  b->down_lora ? d_grad_a[2] : nullptr, b->down_lora ? d_grad_b[2] : nullptr, s);
