@@ -8,8 +8,10 @@
 static std::map<void *, size_t> g_owned;
 static bool g_capturing = false;
 static size_t g_room = (size_t)1 << 40;  // bytes the device still has
+static int g_mallocs = 0, g_frees = 0;
 
 hipError_t hipMalloc(void **p, size_t n) {
+  ++g_mallocs;
   if (g_capturing) return hipErrorStreamCaptureUnsupported;
   if (n > g_room) return hipErrorOutOfMemory;
   static size_t next = 0;  // no address twice
@@ -19,6 +21,7 @@ hipError_t hipMalloc(void **p, size_t n) {
   return hipSuccess;
 }
 hipError_t hipFree(void *p) {
+  ++g_frees;
   auto it = g_owned.find(p);
   if (it == g_owned.end()) return hipErrorInvalidValue;
   g_room += it->second;
@@ -97,7 +100,56 @@ static void eager_growth_frees() {
   EXPECT(g_owned.empty() && b.p == nullptr && b.cap == 0);
 }
 
+// A device without the memory for the larger block: nothing moves, and the
+// refused size costs no further calls to the runtime for a while.
+static void refused_growth_changes_nothing() {
+  DevBuf b;
+  const hipStream_t s = nullptr;
+  std::vector<char *> out;
+  char *const small = carve(1 << 20).bind(b, s)[0];
+  const size_t room = g_room;
+  g_room = (size_t)64 << 20;
+  EXPECT(!carve((size_t)1 << 30).try_bind(b, s, &out));
+  EXPECT(b.p == small && b.cap == 1 << 20 && g_owned.count(small) == 1);
+  const int m = g_mallocs, f = g_frees;
+  for (int i = 0; i < 100; ++i) {
+    EXPECT(!carve((size_t)1 << 30).try_bind(b, s, &out));
+    EXPECT(carve(1 << 20).bind(b, s)[0] == small);  // the fallback
+  }
+  EXPECT(g_mallocs == m && g_frees == f);
+  EXPECT(carve((size_t)32 << 20).try_bind(b, s, &out));  // a smaller one can be had
+  g_room = room;
+  int n = 0;
+  while (n < 1000 && !carve((size_t)1 << 30).try_bind(b, s, &out)) ++n;
+  EXPECT(n < 1000);  // asked for again in the end
+  b.release();
+  EXPECT(g_owned.empty());
+}
+
+// bind() needs its block: where both do not fit, the old one goes first.
+static void needed_growth_frees_first_where_both_do_not_fit() {
+  DevBuf b;
+  const hipStream_t s = nullptr;
+  carve((size_t)40 << 20).bind(b, s);
+  const size_t room = g_room;
+  g_room = (size_t)20 << 20;
+  carve((size_t)50 << 20).bind(b, s);
+  EXPECT(g_owned.size() == 1 && b.cap == (size_t)50 << 20);
+  bool threw = false;
+  try {
+    carve((size_t)80 << 20).bind(b, s);
+  } catch (const qh::GpuError &) {
+    threw = true;
+  }
+  EXPECT(threw);
+  b.release();
+  EXPECT(g_owned.empty());
+  g_room = room;
+}
+
 int main() {
+  refused_growth_changes_nothing();
+  needed_growth_frees_first_where_both_do_not_fit();
   captured_block_outlives_growth();
   kept_blocks_are_bounded();
   eager_growth_frees();

@@ -2,6 +2,7 @@
 // that lays a call's scratch out in them.  Host code only.
 #pragma once
 #include <cstddef>
+#include <cstdint>
 #include <string>
 #include <vector>
 
@@ -32,8 +33,8 @@ inline bool capturing(hipStream_t s) {
 // bound to for as long as it is replayed, and nobody tells the library when
 // that ends: growth frees a block only if no captured call was bound to it,
 // and keeps it until release() otherwise.  A block that takes a kept one's
-// place is at least twice as large, so that the kept ones together stay below
-// the one in use.
+// place is twice as large where the device has that, so that the kept ones
+// together stay below the one in use.
 struct DevBuf {
   void *p = nullptr;
   size_t cap = 0;
@@ -49,23 +50,28 @@ struct DevBuf {
   // For buffers that only blocking host-slice calls use (never captured).
   void *ensure(size_t bytes) {
     if (bytes <= cap) return p;
-    const size_t want = rounded(bytes);
-    retire();
-    check(hipMalloc(&p, want), "hipMalloc");
-    cap = want;
+    hipError_t e = grow(bytes);
+    if (e == hipErrorOutOfMemory && p && !captured) {  // not beside the old block
+      check(hipFree(p), "hipFree");
+      p = nullptr;
+      cap = 0;
+      e = grow(bytes);
+    }
+    check(e, "hipMalloc");
     return p;
   }
-  // False, with the buffer empty, when the device has no such block left.
+  // False, with the buffer as it was, when the device has no such block left.
+  // A size that failed is not asked for again on every call (a failing
+  // hipMalloc waits for the device): the next attempt comes kRetry calls later.
   bool try_ensure(size_t bytes) {
     if (bytes <= cap) return true;
-    const size_t want = rounded(bytes);
-    retire();
-    if (hipMalloc(&p, want) != hipSuccess) {
-      (void)hipGetLastError();
-      p = nullptr;
+    if (bytes >= failed && ++refused < kRetry) return false;
+    refused = 0;
+    if (grow(bytes) != hipSuccess) {
+      if (bytes < failed) failed = bytes;
       return false;
     }
-    cap = want;
+    if (bytes >= failed) failed = SIZE_MAX;
     return true;
   }
   // Notes that a call on `s` is bound to the block.
@@ -79,22 +85,40 @@ struct DevBuf {
     p = nullptr;
     cap = 0;
     captured = false;
+    failed = SIZE_MAX;
+    refused = 0;
   }
 
  private:
-  size_t rounded(size_t bytes) const {
-    if (captured && bytes < 2 * cap) bytes = 2 * cap;
-    return bytes < 256 ? 256 : (bytes + 255) / 256 * 256;
-  }
-  void retire() {
-    if (p && captured) {
-      kept.push_back(p);
-    } else if (p) {
-      check(hipFree(p), "hipFree");
+  static constexpr int kRetry = 256;
+  size_t failed = SIZE_MAX;  // the smallest size that try_ensure could not have
+  int refused = 0;
+
+  // A block for `bytes` in place of the present one, which goes only when the
+  // new one is there.
+  hipError_t grow(size_t bytes) {
+    const auto up = [](size_t n) { return n < 256 ? 256 : (n + 255) / 256 * 256; };
+    size_t want = up(bytes);
+    if (captured) kept.reserve(kept.size() + 1);
+    void *q = nullptr;
+    hipError_t e = hipErrorOutOfMemory;
+    if (captured && want < 2 * cap && (e = hipMalloc(&q, up(2 * cap))) == hipSuccess)
+      want = up(2 * cap);
+    if (!q) e = hipMalloc(&q, want);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return e;
     }
-    p = nullptr;
-    cap = 0;
+    if (captured) {
+      kept.push_back(p);
+    } else if (p && (e = hipFree(p)) != hipSuccess) {
+      (void)hipFree(q);
+      return e;
+    }
+    p = q;
+    cap = want;
     captured = false;
+    return hipSuccess;
   }
 };
 
