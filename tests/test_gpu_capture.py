@@ -49,3 +49,26 @@ def test_replay_after_a_larger_eager_call(M):
         assert torch.equal(_bits(want), _bits(y))
     del gr
     c.close()
+
+
+def test_capture_of_fewer_tokens_than_warmed_up():
+    """The few-token kernel splits K at 33 tokens of this layer and not at 49, so
+    its scratch for 33 exceeds that for 49; the tiles' does not."""
+    import qlora_hip as QH
+    from qlora_hip import device as QD
+    c, d = QH.Context(), QH.Context()
+    W, lora = _layer(QD, c, 2048, 4096, 8)
+    x = torch.randn(49, 4096, device="cuda")
+    y, want = torch.empty(49, 2048, device="cuda"), torch.empty(33, 2048, device="cuda")
+    QD.forward(W, lora, x, 49, y, ctx=c)
+    QD.forward(W, lora, x[:33], 33, want, ctx=d)
+    torch.cuda.synchronize()
+    gr = _capture(lambda: QD.forward(W, lora, x[:33], 33, y, ctx=c))
+    for _ in range(3):
+        y.fill_(float("nan"))
+        gr.replay()
+        torch.cuda.synchronize()
+        # two splits of fp32 products into bf16 parts, 5e-6 of the norm each
+        assert float((y[:33] - want).norm() / want.norm()) < 2e-5
+    del gr
+    c.close(), d.close()

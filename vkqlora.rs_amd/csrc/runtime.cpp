@@ -466,10 +466,14 @@ bool takes_slim(const DevQW &W, const qh_lora *l, const void *x, int xdt, int64_
 // `count` layers, each on its own x (layers with the same x share its
 // preparation); with `beta` y += the result.  False, with nothing launched,
 // where its scratch cannot be had (see Carve::try_bind) or no plan covers the
-// group: the caller runs the layers on the paths with smaller scratch.
+// group: the caller runs the layers on the tile kernels.  Their scratch for
+// these layers is `tile_bytes`, and the buffer grows to that as well: what
+// this kernel needs does not rise with the token count, so a capture of fewer
+// tokens than the calls before it may find too little for it, but not for
+// the tiles, which then need no more than those calls would have.
 bool slim_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora *const *l,
               const void *const *x, int xdt, int64_t M, float *const *y, float *const *t1_out,
-              int beta, hipStream_t s) {
+              int beta, size_t tile_bytes, hipStream_t s) {
   if (count > (size_t)qh::kMaxSlimSegs) return false;
   const int xb = xdt == QH_BF16, n = (int)count;
   int64_t rs[qh::kMaxSlimSegs] = {};
@@ -487,8 +491,10 @@ bool slim_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora *const *l
     ix[i] = c.add(own[i] == i ? pl.xp_bytes[i] : 0);
     ip[i] = c.add(pl.part_floats[i] * 4);
   }
+  Carve both = c;
+  if (tile_bytes > c.total()) both.add(tile_bytes - c.total());
   std::vector<char *> p;
-  if (!c.try_bind(ctx->scratch, s, &p)) return false;
+  if (!both.try_bind(ctx->scratch, s, &p) && !c.try_bind(ctx->scratch, s, &p)) return false;
   qh::SlimIn in[qh::kMaxSlimSegs] = {};
   for (int i = 0; i < n; ++i) {
     in[i].w = W[i], in[i].x = x[i], in[i].y = y[i], in[i].beta = beta;
@@ -539,6 +545,37 @@ void plane_gemm_dev(qh_ctx *ctx, const std::vector<char *> &p, const PlaneSlots 
   timed(ctx, name, s, [&] { return qh::launch_plane_gemm(g, s); });
 }
 
+// What the forward of one layer (M, K, N > 0) runs on the tile kernels, and its
+// scratch.
+struct TileForward {
+  bool fast, bf16;                         // whole 64-element row blocks; on bf16 MFMA
+  bool t1_rank = false, t1_dense = false;  // T1's kernel (else the tile engine)
+  GemmArgs gt1{};
+  DenseOp dt1{};
+  int y_splits;
+  Carve c;
+  size_t i_t1, i_w32, i_p1, i_p2;
+  TileForward(const DevQW &W, const qh_lora *l, const void *x, int xe, int64_t M,
+              const float *t1_out) {
+    const int64_t N = W.rows, K = W.cols, r = l ? (int64_t)l->r : 0;
+    fast = qh::nf4_fast_ok(W);
+    bf16 = fast && qh::bf16_gemm_ok(W, x, K, K);
+    if (l) {
+      t1_rank = qh::rank_gemm_ok(K, r);
+      gt1 = gemm_args(M, r, K, op(x, K, qh::ROWK, xe), op(l->a, K, qh::ROWK, qh::E_F32),
+                      nullptr, r, 1.0f);
+      dt1 = dense_t1(x, xe, M, K, l, nullptr);
+      t1_dense = !t1_rank && dt1.ok();
+      gt1.splits = t1_rank || t1_dense ? 1 : choose_splits(M, r, K);
+    }
+    y_splits = bf16 ? qh::bf16_gemm_splits(M, N, K) : base_splits(M, N, K);
+    i_t1 = c.add(l && !t1_out ? (size_t)M * r * 4 : 0);
+    i_w32 = c.add(fast ? 0 : (size_t)W.n * 4);
+    i_p1 = c.add(!l ? 0 : t1_dense ? dt1.partial_bytes() : partial_floats(gt1) * 4);
+    i_p2 = c.add(y_splits > 1 ? (size_t)y_splits * M * N * 4 : 0);
+  }
+};
+
 // ---- fused forward on device pointers -----------------------------------
 // With `accumulate` y += the result; only the bf16-MFMA path (the one
 // forward_accumulates names) does that, every other path refuses it before
@@ -566,9 +603,9 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
     return;
   }
   if (takes_slim(W, l, x, xdt, M) &&
-      slim_dev(ctx, 1, &W, &l, &x, xdt, M, &y, &t1_out, accumulate ? 1 : 0, s))
+      slim_dev(ctx, 1, &W, &l, &x, xdt, M, &y, &t1_out, accumulate ? 1 : 0,
+               TileForward(W, l, x, xe, M, t1_out).c.total(), s))
     return;
-  const bool fast = qh::nf4_fast_ok(W);
   // Small batches: the MFMA decode kernels (batch <= 16, K % 256 == 0), else
   // the VALU GEMV (batch <= 4, K % 64 == 0); both need 16-byte aligned rows
   // of X and A.
@@ -627,52 +664,34 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
 
   // NF4 weights in whole 64-element row blocks run on bf16 MFMA (the weight
   // as hi / lo bf16 parts); others on the fp32 tile engine
-  const bool bf16 = fast && qh::bf16_gemm_ok(W, x, K, K);
+  TileForward f(W, l, x, xe, M, t1_out);
+  const bool fast = f.fast, bf16 = f.bf16;
   if (!bf16) writes_y("forward_dev: y += on the fp32 tile engine");
-  GemmArgs gt1{}, gm{};
-  const bool t1_rank = lora && qh::rank_gemm_ok(K, r);
-  DenseOp dt1{};
-  bool t1_dense = false;
-  if (lora) {
-    gt1 = gemm_args(M, r, K, op(x, K, qh::ROWK, xe), op(l->a, K, qh::ROWK, qh::E_F32),
-                    nullptr, r, 1.0f);
-    dt1 = dense_t1(x, xe, M, K, l, nullptr);
-    t1_dense = !t1_rank && dt1.ok();
-    gt1.splits = t1_rank || t1_dense ? 1 : choose_splits(M, r, K);
-  }
-  const int y_splits = bf16 ? qh::bf16_gemm_splits(M, N, K) : base_splits(M, N, K);
-  Carve c;
-  const size_t i_t1 = c.add(lora && !t1_out ? (size_t)M * r * 4 : 0);
-  const size_t i_w32 = c.add(fast ? 0 : (size_t)W.n * 4);
-  const size_t i_p1 =
-      c.add(!lora ? 0 : t1_dense ? dt1.partial_bytes() : partial_floats(gt1) * 4);
-  const size_t i_p2 = c.add(y_splits > 1 ? (size_t)y_splits * M * N * 4 : 0);
   // large GEMMs through operand planes where their memory can be had
   bool plane = bf16 && qh::plane_ok(M, N, K);
   Carve cp;
   const PlaneSlots slots(cp, plane, M, N, K, r, xe == qh::E_F32 ? 2 : 1);
   std::vector<char *> pp;
   plane = plane && cp.try_bind(ctx->planes, s, &pp);
-  auto p = c.bind(ctx->scratch, s);
-  float *t1 = lora ? (t1_out ? t1_out : (float *)p[i_t1]) : nullptr;
+  auto p = f.c.bind(ctx->scratch, s);
+  float *t1 = lora ? (t1_out ? t1_out : (float *)p[f.i_t1]) : nullptr;
 
-  if (lora && t1_rank) {
+  if (lora && f.t1_rank) {
     timed(ctx, "t1_gemm", s, [&] {
       return qh::launch_rank_gemm(x, xe == qh::E_BF16, K, l->a, 0, K, t1, r, M, K, r, 1.0f, s);
     });
-  } else if (lora && t1_dense) {
-    dt1.c = t1;
-    timed(ctx, "t1_gemm", s, [&] { return dt1.run((float *)p[i_p1], s); });
+  } else if (lora && f.t1_dense) {
+    f.dt1.c = t1;
+    timed(ctx, "t1_gemm", s, [&] { return f.dt1.run((float *)p[f.i_p1], s); });
   } else if (lora) {
-    gt1.C = t1;
-    timed(ctx, "t1_gemm", s, [&] { return qh::launch_gemm(gt1, (float *)p[i_p1], s); });
+    f.gt1.C = t1;
+    timed(ctx, "t1_gemm", s, [&] { return qh::launch_gemm(f.gt1, (float *)p[f.i_p1], s); });
   }
   Operand B;
-  DevQW qw = W;
   if (fast) {
     B = op(W.codes, K, qh::ROWK, qh::E_NF4);
   } else {
-    float *w32 = (float *)p[i_w32];
+    float *w32 = (float *)p[f.i_w32];
     timed(ctx, "dequantize", s, [&] { return qh::launch_dequantize(W, w32, s); });
     B = op(w32, K, qh::ROWK, qh::E_F32);
   }
@@ -693,20 +712,20 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
     if (lora) q.A2 = t1, q.lda2 = r, q.B2 = l->b, q.ldb2 = r, q.b2scale = sc, q.K2 = r;
     timed(ctx, "forward_gemm_bf16", s,
           [&] {
-            return qh::launch_gemm_bf16(b, qh::ROWK, xe == qh::E_F32, y_splits,
-                                        (float *)p[i_p2], s);
+            return qh::launch_gemm_bf16(b, qh::ROWK, xe == qh::E_F32, f.y_splits,
+                                        (float *)p[f.i_p2], s);
           });
     return;
   }
-  gm = gemm_args(M, N, K, op(x, K, qh::ROWK, xe), B, y, N, 1.0f);
-  gm.qw = qw;
+  GemmArgs gm = gemm_args(M, N, K, op(x, K, qh::ROWK, xe), B, y, N, 1.0f);
+  gm.qw = W;
   if (lora) {
     gm.K2 = r;
     gm.A2 = op(t1, r, qh::ROWK, qh::E_F32);
     gm.B2 = op(l->b, r, qh::ROWK, qh::E_F32, sc);
   }
-  gm.splits = y_splits;
-  timed(ctx, "forward_gemm", s, [&] { return qh::launch_gemm(gm, (float *)p[i_p2], s); });
+  gm.splits = f.y_splits;
+  timed(ctx, "forward_gemm", s, [&] { return qh::launch_gemm(gm, (float *)p[f.i_p2], s); });
 }
 
 // y += forward(x): in the bf16 GEMM's epilogue (or its split-K reduction)
@@ -966,18 +985,27 @@ void forward_shared_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora
                         const void *x, int xdt, size_t batch, float *const *y,
                         float *const *t1_out, hipStream_t s) {
   const int64_t M = (int64_t)batch, K = W[0].cols;
+  const int xe = xdt == QH_BF16 ? qh::E_BF16 : qh::E_F32;
   bool slim = count <= (size_t)qh::kMaxSlimSegs;
   for (size_t i = 0; i < count && slim; ++i) slim = takes_slim(W[i], l[i], x, xdt, M);
+  const bool shared = shared_ok(count, W, l, x, nullptr, M);
   if (slim) {
     const void *const xs[qh::kMaxSlimSegs] = {x, x, x, x};
-    if (slim_dev(ctx, count, W, l, xs, xdt, M, y, t1_out, 0, s)) return;
+    size_t tile_bytes = 0;
+    for (size_t i = 0; i < count; ++i) {
+      const float *t1i = t1_out ? t1_out[i] : nullptr;
+      if (shared)
+        tile_bytes += l[i] && !t1i ? (size_t)M * l[i]->r * 4 + 256 : 0;
+      else
+        tile_bytes = std::max(tile_bytes, TileForward(W[i], l[i], x, xe, M, t1i).c.total());
+    }
+    if (slim_dev(ctx, count, W, l, xs, xdt, M, y, t1_out, 0, tile_bytes, s)) return;
   }
-  if (!shared_ok(count, W, l, x, nullptr, M)) {
+  if (!shared) {
     for (size_t i = 0; i < count; ++i)
       forward_dev(ctx, W[i], l[i], x, xdt, batch, y[i], t1_out ? t1_out[i] : nullptr, s);
     return;
   }
-  const int xe = xdt == QH_BF16 ? qh::E_BF16 : qh::E_F32;
   Carve c;
   size_t it[kMaxShared];
   for (size_t i = 0; i < count; ++i)
