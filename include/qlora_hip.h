@@ -265,11 +265,13 @@ QH_API qh_status qh_qlora_backward_dev(qh_ctx *ctx, const qh_qweight *w,
                                        float *d_grad_b, void *stream);
 /* Allocation-free fused backward: no counterpart in the reference.  For
  * callers that cannot allocate device memory (code under HIP graph capture,
- * tight serving loops, harnesses that forbid hipMalloc).  Arguments, results
- * and kernels are those of qh_qlora_backward_dev, but its scratch (T1 when
- * d_t1 is NULL, Ds = s.dY.B, split-K partial sums) lives in a fixed region of
- * QH_NOALLOC_SCRATCH_BYTES that each GPU holds from the first context created
- * on it until the process ends; the call allocates nothing.  A call that
+ * tight serving loops, harnesses that forbid hipMalloc).  Arguments and
+ * results, bit for bit, are those of qh_qlora_backward_dev, but its scratch
+ * (T1 when d_t1 is NULL, Ds = s.dY.B, split-K partial sums) lives in a fixed
+ * region of QH_NOALLOC_SCRATCH_BYTES that each GPU holds from the first context
+ * created on it until the process ends; the call allocates nothing.  So it
+ * has no room for the operand planes of large input gradients, and computes
+ * those at the speed of the kernel without them.  A call that
  * would need more scratch fails with QH_ERR_INVALID_CONFIG before any
  * launch.  Every call on one GPU shares that GPU's region: calls that
  * overlap on one GPU (other streams, other contexts, other threads) race,

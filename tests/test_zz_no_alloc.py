@@ -1,7 +1,8 @@
 """GPU parity of the allocation-free backward (qh_qlora_backward_dev_noalloc)
-against qh_qlora_backward_dev, through the C ABI: the same kernels with the
+against qh_qlora_backward_dev, through the C ABI: the same sums with the
 scratch in the library's fixed per-GPU region, so grad_x, grad_A and grad_B
-must be the same bits.  Two calls in a row, the second smaller (the region
+must be the same bits, also where the input gradient of the other entry point
+goes through operand planes.  Two calls in a row, the second smaller (the region
 keeps the first call's contents), with and without a T1 from the forward,
 fp32 and bf16 activations, split-K partials in the region; a call that
 needs more than the region is refused before any launch."""
@@ -65,6 +66,30 @@ def test_noalloc_backward_same_bits_two_calls(ctx, act, with_t1):
         for gname, gv, wv in zip(("grad_x", "grad_a", "grad_b"), got, want):
             assert not torch.isnan(wv).any(), gname
             assert torch.equal(gv.view(torch.int32), wv.view(torch.int32)), gname
+
+
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,K,M,planes", [
+    (2056, 4160, 1100, True),   # through operand planes, ragged in every direction
+    (768, 128, 20000, False),   # few columns, many tokens: k_nf4_bf16 splits the reduction
+])
+def test_noalloc_backward_same_bits_large_calls(ctx, N, K, M, planes, act):
+    from qlora_hip import device as QD
+    g = torch.Generator(device="cuda").manual_seed(N + K + M)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    W = QD.DeviceWeight.quantize(rnd(N, K) * 0.02, 64, True, ctx=ctx)
+    lora = QD.lora_struct(rnd(16, K) * 0.02, rnd(N, 16) * 0.01, 16, 16.0)
+    x, dy = rnd(M, K).to(act), rnd(M, N).to(act)
+    ctx.set_timing(True)
+    want = _backward(QD, ctx, ctx.lib.qh_qlora_backward_dev, W, lora, x, dy, None, M)
+    torch.cuda.synchronize()
+    rep = ctx.timing_report(reset=True)
+    ctx.set_timing(False)
+    assert ("planes" in rep) == planes, rep
+    got = _backward(QD, ctx, ctx.lib.qh_qlora_backward_dev_noalloc, W, lora, x, dy, None, M)
+    torch.cuda.synchronize()
+    for gname, gv, wv in zip(("grad_x", "grad_a", "grad_b"), got, want):
+        assert torch.equal(gv.view(torch.int32), wv.view(torch.int32)), gname
 
 
 def test_noalloc_backward_refuses_oversized_calls(ctx):

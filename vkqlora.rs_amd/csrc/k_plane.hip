@@ -519,9 +519,12 @@ int plane_bm(int64_t M, int64_t N) {
 // Worth its pass over the operands where the output has more than half a round
 // of 128 x 256 tiles (measured, fp32 / bf16 X): 129 tiles 1.24 / 1.28 times as fast
 // as the other tiles, 192 1.34 / 1.28, 256 and more 1.05 to 1.4, 128 1.02 / 0.94,
-// 96 0.97 / 0.94, 64 0.7; K of 512 or more, and at most 2 GiB of planes.
+// 96 0.97 / 0.94, 64 0.7; K of 512 or more, and at most 2 GiB of planes.  What
+// k_nf4_bf16 splits (at most 128 columns, up to 21760 rows) stays there: its
+// bits are those of the allocation-free backward, which takes no planes.
 bool plane_ok(int64_t M, int64_t N, int64_t K) {
-  return up(M, 128) * up(N, 256) > 128 && K >= 512 && M < (1 << 24) && N < (1 << 24) &&
+  return up(M, 128) * up(N, 256) > 128 && K >= 512 && bf16_gemm_splits(M, N, K) == 1 &&
+         M < (1 << 24) && N < (1 << 24) &&
          K < (1 << 24) && plane_a_bytes(M, K, 2) + plane_b_bytes(N, K) <= (size_t)2 << 30;
 }
 

@@ -1831,7 +1831,8 @@ qh_status qh_qlora_backward_dev_noalloc(qh_ctx *ctx, const qh_qweight *w, const 
   qh_status st = validate_backward_dev(w, lora, d_x, d_dy, act_dtype, batch, d_grad_x,
                                        d_grad_a, d_grad_b);
   if (st != QH_OK) return st;
-  // The same plan as qh_qlora_backward_dev; its scratch must fit the region.
+  // The plan of qh_qlora_backward_dev without operand planes (the same bits);
+  // its scratch must fit the region.
   size_t need = 0;
   backward_dev(ctx, make_devqw(*w), lora, d_x, d_dy, act_dtype, batch, d_t1, d_grad_x,
                d_grad_a, d_grad_b, nullptr, nullptr, &need);
