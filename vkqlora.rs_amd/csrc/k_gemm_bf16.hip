@@ -712,10 +712,12 @@ hipError_t run_bf16(const Bf16GemmArgs &g0, int splits, float *partial, hipStrea
 
 // Block shape and reduction splits by problem size.
 //  large:  256 x 256 or 256 x 128 tiles, 8 waves, for problems with at least
-//          256 tiles of 256 x 256 (MFMA-bound); such a problem comes here
-//          only where the operand planes of k_plane.hip cannot have their
-//          scratch (4096^3 in fp32 400 us here, 350 with planes), or in a
-//          group that also holds smaller layers;
+//          256 tiles of 256 x 256 (MFMA-bound); most of these go through the
+//          operand planes of k_plane.hip instead (4096^3 in fp32 400 us here,
+//          350 there).  Here come those that planes would not speed up (few
+//          columns or rows against the other sizes, K below 512), whose planes
+//          pass 2 GiB or cannot have their memory (a full device, a capture
+//          before a warm-up), groups, and the allocation-free backward;
 //  medium: 128 x 128 tiles, 8 waves, loads two steps ahead, two 32-wide
 //          sub-steps per barrier (one when there are more tiles than CUs,
 //          so that two blocks share a CU), for 160 or more tiles of
@@ -754,6 +756,13 @@ Plan plan_for(int64_t M, int64_t N, int64_t K) {
   return Plan{tier, sp < 1 ? 1 : (int)sp};
 }
 
+// Large tier: 256 x 256 tiles where they fill at least 3/4 of their rounds of
+// 256 workgroups, else 256 x 128.
+bool wide_tiles(int64_t M, int64_t N) {
+  const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256), waves = (t256 + 255) / 256;
+  return t256 >= 192 && (double)t256 / (double)(waves * 256) >= 0.75;
+}
+
 template <int WF, int XF, int KIND>
 hipError_t pick(const Bf16GemmArgs &g, int splits, float *partial, hipStream_t s) {
   const Plan pl = plan_for(g.M, g.N, g.K);
@@ -764,10 +773,7 @@ hipError_t pick(const Bf16GemmArgs &g, int splits, float *partial, hipStream_t s
       return run_bf16<CfgM1, WF, XF, KIND>(g, splits, partial, s);
     return run_bf16<CfgM, WF, XF, KIND>(g, splits, partial, s);
   }
-  const int64_t t256 = ((g.M + 255) / 256) * ((g.N + 255) / 256);
-  const int64_t waves = (t256 + 255) / 256;
-  const bool wide = t256 >= 192 && (double)t256 / (double)(waves * 256) >= 0.75;
-  return wide ? run_bf16<CfgL256, WF, XF, KIND>(g, 1, nullptr, s)
+  return wide_tiles(g.M, g.N) ? run_bf16<CfgL256, WF, XF, KIND>(g, 1, nullptr, s)
               : run_bf16<CfgL128, WF, XF, KIND>(g, 1, nullptr, s);
 }
 
@@ -1041,6 +1047,36 @@ bool bf16_gemm_ok(const DevQW &w, const void *a, int64_t lda, int64_t K) {
 }
 
 int bf16_gemm_splits(int64_t M, int64_t N, int64_t K) { return plan_for(M, N, K).splits; }
+
+// Fitted to some 1500 forwards and input gradients (16 to 65536 rows and columns,
+// K 320 to 11008): within 6 % rms, 4 % above 40 us.  A step of 32 k costs what the
+// rounds of workgroups take at full and at partial occupancy (two blocks of the
+// medium tier fit a CU where it has more tiles than CUs, four small ones do),
+// plus the tiles' share of operand traffic.
+double bf16_gemm_us(int64_t M, int64_t N, int64_t K, bool f32, bool split) {
+  const Plan p = plan_for(M, N, K);
+  const auto up = [](int64_t a, int64_t b) { return (double)((a + b - 1) / b); };
+  const int64_t steps = (K + kBK - 1) / kBK;
+  const double mn = (double)M * (double)N * 1e-6;
+  if (p.tier == kLarge) {
+    const bool wide = wide_tiles(M, N);
+    const double t = up(M, 256) * up(N, wide ? 256 : 128), R = up((int64_t)t, 256);
+    const double step = wide ? f32 ? 1.49 * R + 0.0042 * t : 1.15 * R + 0.0026 * t
+                             : f32 ? 1.28 * R + 0.0011 * t : 0.96 * R + 0.00055 * t;
+    return (wide ? 3.5 + 2 * R : 9 + R) + (double)steps * step + (f32 ? 0.45 : 0.35) * mn;
+  }
+  const int sp = split ? p.splits : 1;
+  const double tile = p.tier == kMedium ? 128 : 64, t = up(M, (int64_t)tile) * up(N, (int64_t)tile);
+  const double wg = t * sp / 256, R = up((int64_t)t * sp, 256), ks = up(steps, sp);
+  if (p.tier == kSmall)
+    return 3.65 + ks * (f32 ? 0.53 + 0.145 * (R - 1) + 0.11 * wg : 0.425 + 0.108 * (R - 1) + 0.083 * wg) +
+           (sp > 1 ? 2.1 + 2 * sp * mn : 0);
+  if (t <= 256)
+    return 5.6 + ks * (f32 ? 0.95 + 0.9 * (R - 1) + 0.09 * wg : 0.8 + 0.72 * (R - 1)) +
+           (sp > 1 ? 0.18 + 2.85 * sp * mn : 0) + (f32 ? 0.7 : 0.5) * mn;
+  const double R2 = up((int64_t)t * sp, 512);
+  return 6.9 + ks * (0.295 * R2 + (f32 ? 0.43 * R + 0.3175 * wg : 0.33 * R + 0.16 * wg)) + 0.23 * mn;
+}
 
 hipError_t launch_gemm_bf16(const Bf16GemmArgs &g, int w_form, int a_f32, int splits,
                             float *partial, hipStream_t s) {

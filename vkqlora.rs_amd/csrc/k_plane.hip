@@ -514,18 +514,44 @@ int plane_bm(int64_t M, int64_t N) {
   return best;
 }
 
+// About what the planes and the GEMM take (us): their bytes, the rounds of
+// tiles, the tiles' operand traffic and the output.  Fitted to the same calls as
+// bf16_gemm_us, 5 to 6 % rms; the constant is 3 us above the fit, for the calls
+// below 40 us.
+double plane_us(int64_t M, int64_t N, int64_t K, bool f32) {
+  const int bm = plane_bm(M, N);
+  const double m = (double)M, n = (double)N, k = (double)K;
+  const double t = (double)(up(M, bm) * up(N, 256)), R = (double)up((int64_t)t, 256);
+  if (f32)
+    return 13 + (1.36 * m + 0.97 * n) * k * 1e-6 + k * (R * (bm + 24) * 107e-6 + t * bm * 54e-8) +
+           m * n * 0.48e-6 + R * bm * 0.0135;
+  return 15.7 + (0.62 * m + 1.03 * n) * k * 1e-6 + k * (R * (bm + 24) * 105e-6 + t * bm * 19.5e-8) +
+         m * n * 1.05e-6 - R * bm * 0.021;
+}
+
 }  // namespace
 
-// Worth its pass over the operands where the output has more than half a round
-// of 128 x 256 tiles (measured, fp32 / bf16 X): 129 tiles 1.24 / 1.28 times as fast
-// as the other tiles, 192 1.34 / 1.28, 256 and more 1.05 to 1.4, 128 1.02 / 0.94,
-// 96 0.97 / 0.94, 64 0.7; K of 512 or more, and at most 2 GiB of planes.  What
-// k_nf4_bf16 splits (at most 128 columns, up to 21760 rows) stays there: its
-// bits are those of the allocation-free backward, which takes no planes.
-bool plane_ok(int64_t M, int64_t N, int64_t K) {
+// Planes where their estimate is below that of k_nf4_bf16, in the range measured:
+// more than half a round of 128 x 256 tiles and K of 512 or more, at most 2 GiB of
+// planes (the LoRA term of rank r included).  The pass over the operands costs (8 or 4 bytes) x rows + 4.5 bytes x columns per k,
+// whatever the product, and columns are padded to 256, so that narrow outputs
+// and few rows lose: fp32 20000 x 192 over 2048 188 us against 150, 64 x 128256
+// over 4096 888 against 448, 2048 x 4096 over 512 39 against 37; they win from
+// about 576 columns and 400 rows at K of 1536 (8192 x 576 87 against 97), 1.2
+// times as fast on the geometric mean of the sizes taken here, 1.4 at 1100 x 4096
+// over 4096.  Of 1456 calls measured, fp32 and bf16, forward and input gradient,
+// 719 are taken, 9 of them slower by more than 3 % (at most 7); 125 of the
+// others would be faster by more than 5 % (all of these shapes: 421 slower, up
+// to 3.1 times).  What k_nf4_bf16 splits (at most 128 columns, up to 21760 rows)
+// stays there: its bits are those of the allocation-free backward, which takes
+// no planes.
+bool plane_ok(int64_t M, int64_t N, int64_t K, int64_t r, bool f32) {
   return up(M, 128) * up(N, 256) > 128 && K >= 512 && bf16_gemm_splits(M, N, K) == 1 &&
-         M < (1 << 24) && N < (1 << 24) &&
-         K < (1 << 24) && plane_a_bytes(M, K, 2) + plane_b_bytes(N, K) <= (size_t)2 << 30;
+         M < (1 << 24) && N < (1 << 24) && K < (1 << 24) && r < (1 << 24) &&
+         plane_a_bytes(M, K, 2) + plane_b_bytes(N, K) + plane_a_bytes(M, r, 2) +
+                 plane_b_bytes(N, r) <=
+             (size_t)2 << 30 &&
+         plane_us(M, N, K, f32) < 0.98 * bf16_gemm_us(M, N, K, f32, true);
 }
 
 size_t plane_a_bytes(int64_t M, int64_t K, int parts) {

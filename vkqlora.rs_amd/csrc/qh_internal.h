@@ -120,6 +120,9 @@ bool bf16_gemm_ok(const DevQW &w, const void *a, int64_t lda, int64_t K);
 // Reduction splits the bf16 kernels use for (M x N) outputs over K: > 1
 // needs splits * M * N floats of partial sums.
 int bf16_gemm_splits(int64_t M, int64_t N, int64_t K);
+// About what they take for it (us), with fp32 or bf16 activations; `split`: in
+// those splits (grouped forwards run in one).
+double bf16_gemm_us(int64_t M, int64_t N, int64_t K, bool f32, bool split);
 hipError_t launch_gemm_bf16(const Bf16GemmArgs &g, int w_form, int a_f32, int splits,
                             float *partial, hipStream_t s);
 // Dense C = alpha sum_k A(m, k) B(n, k) on bf16 MFMA (fp32 operands as hi +
@@ -265,8 +268,9 @@ struct PlaneSrc {
   DevQW w;
   void *dst;
 };
-// Whether an M x N output over K goes through planes.
-bool plane_ok(int64_t M, int64_t N, int64_t K);
+// Whether an M x N output over K with an adapter of rank r (0: none) and fp32 or
+// bf16 activations goes through planes.
+bool plane_ok(int64_t M, int64_t N, int64_t K, int64_t r, bool f32);
 // Bytes of an A operand's (M rows) and a B operand's (N rows) planes.
 size_t plane_a_bytes(int64_t M, int64_t K, int parts);
 size_t plane_b_bytes(int64_t N, int64_t K);

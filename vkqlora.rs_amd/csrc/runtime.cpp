@@ -668,7 +668,7 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
   const bool fast = f.fast, bf16 = f.bf16;
   if (!bf16) writes_y("forward_dev: y += on the fp32 tile engine");
   // large GEMMs through operand planes where their memory can be had
-  bool plane = bf16 && qh::plane_ok(M, N, K);
+  bool plane = bf16 && qh::plane_ok(M, N, K, r, xe == qh::E_F32);
   Carve cp;
   const PlaneSlots slots(cp, plane, M, N, K, r, xe == qh::E_F32 ? 2 : 1);
   std::vector<char *> pp;
@@ -843,7 +843,7 @@ void backward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
   }
   // the input gradient through operand planes where their memory can be had
   // (never in the fixed region, whose bound is part of the interface)
-  bool plane = bf16 && !src && qh::plane_ok(M, K, N);
+  bool plane = bf16 && !src && qh::plane_ok(M, K, N, r, a32);
   Carve cp;
   const PlaneSlots slots(cp, plane, M, K, N, r, a32 ? 2 : 1);
   std::vector<char *> pp;
@@ -958,13 +958,15 @@ void backward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
 constexpr size_t kMaxShared = 3;  // members: 2 rank jobs each in one launch
 
 bool shared_ok(size_t count, const DevQW *W, const qh_lora *const *l, const void *x,
-               const void *const *dy, int64_t M) {
+               const void *const *dy, int64_t M, bool f32) {
   if (count < 2 || count > kMaxShared || count > (size_t)qh::kMaxBf16Segs) return false;
   const int64_t K = W[0].cols;
   // members that are all large GEMMs run through operand planes one by one
   bool planes = true;
-  for (size_t i = 0; i < count; ++i)
-    planes = planes && (dy ? qh::plane_ok(M, K, W[i].rows) : qh::plane_ok(M, W[i].rows, K));
+  for (size_t i = 0; i < count; ++i) {
+    const int64_t N = W[i].rows, r = l[i] ? (int64_t)l[i]->r : 0;
+    planes = planes && (dy ? qh::plane_ok(M, K, N, r, f32) : qh::plane_ok(M, N, K, r, f32));
+  }
   if (planes) return false;
   for (size_t i = 0; i < count; ++i) {
     if (W[i].cols != K || W[i].rows == 0 || W[i].kind != W[0].kind) return false;
@@ -988,7 +990,7 @@ void forward_shared_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora
   const int xe = xdt == QH_BF16 ? qh::E_BF16 : qh::E_F32;
   bool slim = count <= (size_t)qh::kMaxSlimSegs;
   for (size_t i = 0; i < count && slim; ++i) slim = takes_slim(W[i], l[i], x, xdt, M);
-  const bool shared = shared_ok(count, W, l, x, nullptr, M);
+  const bool shared = shared_ok(count, W, l, x, nullptr, M, xe == qh::E_F32);
   if (slim) {
     const void *const xs[qh::kMaxSlimSegs] = {x, x, x, x};
     size_t tile_bytes = 0;
@@ -1048,7 +1050,7 @@ void backward_shared_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lor
                          const float *const *t1_in, float *gx, float *const *ga,
                          float *const *gb, hipStream_t s) {
   const int64_t M = (int64_t)batch, K = W[0].cols;
-  if (!shared_ok(count, W, l, x, dy, M)) {
+  if (!shared_ok(count, W, l, x, dy, M, adt != QH_BF16)) {
     // members after the first add their input gradient into gx: in the
     // GEMM's epilogue where the path allows it, else through a separate add
     for (size_t i = 0; i < count; ++i) {
