@@ -126,6 +126,35 @@ def test_calls_that_planes_slow_down_stay_off_them(ctx, N, K, M):
         assert "planes" not in fwd and "planes" not in bwd, (fwd, bwd)
 
 
+@pytest.mark.parametrize("Ns,K,M,planes", [
+    ((4352, 4352, 4352), 1088, 1024, (False, False)),  # one launch fills its rounds better
+    ((2304, 2304, 2304), 2048, 2048, (False, False)),
+    ((4096, 4096), 4096, 1100, (True, True)),
+])
+def test_groups_take_the_faster_of_planes_and_one_launch(ctx, Ns, K, M, planes):
+    from qlora_hip import device as QD
+    rnd = lambda *s: torch.randn(*s, device="cuda")  # noqa: E731
+    Ls = [(QD.DeviceWeight.quantize(rnd(N, K) * 0.02, 64, True, ctx=ctx), None) for N in Ns]
+    x, ys = rnd(M, K), [torch.empty(M, N, device="cuda") for N in Ns]
+    dys, gx = [rnd(M, N) for N in Ns], torch.empty(M, K, device="cuda")
+    ctx.set_timing(True)
+    QD.forward_shared(Ls, x, M, ys, ctx=ctx)
+    fwd = ctx.timing_report(reset=True)
+    QD.backward_shared(Ls, x, dys, M, gx, ctx=ctx)
+    torch.cuda.synchronize()
+    bwd = ctx.timing_report(reset=True)
+    ctx.set_timing(False)
+    for rep, name, p in ((fwd, "forward_gemm_bf16", planes[0]), (bwd, "grad_x_gemm_bf16", planes[1])):
+        assert ("planes" in rep) == p and rep[name][0] == (len(Ns) if p else 1), rep
+    want = 0
+    for (W, _), y, dy in zip(Ls, ys, dys):
+        wd = W.dequantize(ctx=ctx).view(W.rows, K).double()
+        w = x.double() @ wd.T
+        assert float((y - w).norm() / w.norm()) < 2e-5
+        want = want + dy.double() @ wd
+    assert float((gx - want).norm() / want.norm()) < 2e-5
+
+
 def test_plane_shared_sum_and_residual(ctx):
     """Two layers that both take planes: the second adds its input gradient to
     the first's."""

@@ -514,6 +514,8 @@ int plane_bm(int64_t M, int64_t N) {
   return best;
 }
 
+}  // namespace
+
 // About what the planes and the GEMM take (us): their bytes, the rounds of
 // tiles, the tiles' operand traffic and the output.  Fitted to the same calls as
 // bf16_gemm_us, 5 to 6 % rms; the constant is 3 us above the fit, for the calls
@@ -528,8 +530,6 @@ double plane_us(int64_t M, int64_t N, int64_t K, bool f32) {
   return 15.7 + (0.62 * m + 1.03 * n) * k * 1e-6 + k * (R * (bm + 24) * 105e-6 + t * bm * 19.5e-8) +
          m * n * 1.05e-6 - R * bm * 0.021;
 }
-
-}  // namespace
 
 // Planes where their estimate is below that of k_nf4_bf16, in the range measured:
 // more than half a round of 128 x 256 tiles and K of 512 or more, at most 2 GiB of

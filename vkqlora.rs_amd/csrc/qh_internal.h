@@ -271,6 +271,8 @@ struct PlaneSrc {
 // Whether an M x N output over K with an adapter of rank r (0: none) and fp32 or
 // bf16 activations goes through planes.
 bool plane_ok(int64_t M, int64_t N, int64_t K, int64_t r, bool f32);
+// About what they then take (us).
+double plane_us(int64_t M, int64_t N, int64_t K, bool f32);
 // Bytes of an A operand's (M rows) and a B operand's (N rows) planes.
 size_t plane_a_bytes(int64_t M, int64_t K, int parts);
 size_t plane_b_bytes(int64_t N, int64_t K);

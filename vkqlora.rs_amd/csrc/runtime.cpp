@@ -961,13 +961,23 @@ bool shared_ok(size_t count, const DevQW *W, const qh_lora *const *l, const void
                const void *const *dy, int64_t M, bool f32) {
   if (count < 2 || count > kMaxShared || count > (size_t)qh::kMaxBf16Segs) return false;
   const int64_t K = W[0].cols;
-  // members that are all large GEMMs run through operand planes one by one
+  // Members that are all large GEMMs run through operand planes one by one where
+  // that is faster than one launch of the group (by both estimates, see plane_ok):
+  // three forwards of 1024 x 4352 over 640 in fp32 take 120 us through planes and 78
+  // in one launch, of 2048 x 4096 over 4096 545 and 609, their input gradients 589
+  // and 745.
   bool planes = true;
-  for (size_t i = 0; i < count; ++i) {
+  double us = 0;
+  int64_t sum = 0;
+  for (size_t i = 0; i < count && planes; ++i) {
     const int64_t N = W[i].rows, r = l[i] ? (int64_t)l[i]->r : 0;
-    planes = planes && (dy ? qh::plane_ok(M, K, N, r, f32) : qh::plane_ok(M, N, K, r, f32));
+    planes = dy ? qh::plane_ok(M, K, N, r, f32) : qh::plane_ok(M, N, K, r, f32);
+    us += dy ? qh::plane_us(M, K, N, f32) : qh::plane_us(M, N, K, f32);
+    sum += N;
   }
-  if (planes) return false;
+  if (planes && us < 0.98 * (dy ? qh::bf16_gemm_us(M, K, sum, f32, true)
+                                : qh::bf16_gemm_us(M, sum, K, f32, false)))
+    return false;
   for (size_t i = 0; i < count; ++i) {
     if (W[i].cols != K || W[i].rows == 0 || W[i].kind != W[0].kind) return false;
     if (!qh::nf4_fast_ok(W[i]) || !qh::bf16_gemm_ok(W[i], x, K, K)) return false;
