@@ -546,7 +546,7 @@ double plane_us(int64_t M, int64_t N, int64_t K, bool f32) {
 // stays there: its bits are those of the allocation-free backward, which takes
 // no planes.
 bool plane_ok(int64_t M, int64_t N, int64_t K, int64_t r, bool f32) {
-  return up(M, 128) * up(N, 256) > 128 && K >= 512 && bf16_gemm_splits(M, N, K) == 1 &&
+  return M >= 288 && up(M, 128) * up(N, 256) > 128 && K >= 512 && bf16_gemm_splits(M, N, K) == 1 &&
          M < (1 << 24) && N < (1 << 24) && K < (1 << 24) && r < (1 << 24) &&
          plane_a_bytes(M, K, 2) + plane_b_bytes(N, K) + plane_a_bytes(M, r, 2) +
                  plane_b_bytes(N, r) <=
