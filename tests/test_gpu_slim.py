@@ -124,6 +124,31 @@ def test_slim_refused_forms_take_the_general_path(ctx):
         assert nerr(L["y"].cpu().numpy(), want, K, L["x"], L["wd"]) < 5e-5
 
 
+@pytest.mark.parametrize("Ns,K,r,M", [
+    ((136,), 2560, 0, 468),             # no adapter: the tiles are one short launch
+    ((13904,), 768, 64, 126),           # rows enough to fill the tiles' one round
+    ((1960, 1960, 640), 576, 0, 299),   # a group that the tiles run in one launch
+    ((1752, 1752), 448, 8, 300),
+])
+def test_calls_that_slim_slows_down_stay_on_the_tiles(ctx, Ns, K, r, M):
+    from qlora_hip import device as QD
+    for act in (torch.float32, torch.bfloat16):
+        Ls, x = [], None
+        for N in Ns:
+            Ls.append(_layer(QD, ctx, O.Rng(N + K), N, K, r, M, act, True, x))
+            x = Ls[0]["x"]
+        ctx.set_timing(True)
+        if len(Ns) == 1:
+            QD.forward(Ls[0]["W"], Ls[0]["lora"], Ls[0]["tx"], M, Ls[0]["y"], ctx=ctx)
+        else:
+            QD.forward_shared([(L["W"], L["lora"]) for L in Ls], Ls[0]["tx"], M,
+                              [L["y"] for L in Ls], ctx=ctx)
+        torch.cuda.synchronize()
+        rep = ctx.timing_report(reset=True)
+        ctx.set_timing(False)
+        assert "forward_slim" not in rep, rep
+
+
 def test_slim_under_capture(ctx):
     """A captured forward replays to the eager bits; so does one on a context
     whose scratch would have to grow, where a path that needs none takes it."""

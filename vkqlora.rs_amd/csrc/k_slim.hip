@@ -627,20 +627,15 @@ hipError_t run_slim(const SlimArgs &A, dim3 grid, uint32_t lds, hipStream_t st) 
 
 }  // namespace
 
-// The forward's calls that this path takes: whole 64-element blocks a row,
-// rank at most 64, 16-byte aligned codes, X and A; and, as measured against
-// the GEMM tiles,
+// The forward's calls that this path can take: whole 64-element blocks a row,
+// rank at most 64, 16-byte aligned codes, X and A; and the range in which it was
+// timed against the GEMM tiles (within it SlimPlan::us decides):
 //  * 17 tokens or more (below, the decode kernels),
-//  * up to 512 tokens while tokens x rows stay within 3M (fp32) or 6M (bf16):
-//    14336 x 4096 in fp32 at 160 tokens 110 against 154 us, at 256 (3.7M)
-//    166 against 156; bf16 at 384 tokens (5.5M) 161 against 172, at 512 201
-//    against 188; 11008 x 4096 in fp32 at 256 130 against 155,
-//  * with K below 1024 up to 384 tokens; a short K has few units a wave against
-//    a workgroup's fixed 8 us: below 768 up to 600k outputs (1536 x 576 at 384
-//    tokens 19.5 against 22.0 us, at 512 27.4 against 23.2), below 512 up to
-//    350k (1752 x 320 in fp32 at 192 tokens 15.0 against 16.0, at 256 17.4
-//    against 16.1), below 320 not at all (1752 x 192 14 against 13 at any
-//    count).
+//  * up to 512 tokens while tokens x rows stay within 3M (fp32) or 6M (bf16), or
+//    up to 48 tokens of any row count: 128256 x 4096 at 20 tokens in fp32 161 us
+//    against 414, 33000 x 2048 at 48 48 against 112,
+//  * with K below 1024 up to 384 tokens; below 768 up to 600k outputs, below 512
+//    up to 350k, below 320 none (1752 x 192 14 us against 13 at any count).
 bool slim_ok(const DevQW &w, const void *x, int x_bf16, const float *a, int64_t M, int64_t r) {
   auto al = [](const void *p) { return (((uintptr_t)p) & 15) == 0; };
   if (M < 17 || M > (w.cols < 1024 ? 384 : 512) || w.cols < 320) return false;
@@ -661,7 +656,15 @@ bool slim_ok(const DevQW &w, const void *x, int x_bf16, const float *a, int64_t 
 //    (4 x 16 rows: measured 4200 cycles for R = 2, 6500 for R = 3 at 48
 //    fp32 tokens),
 // plus 15000 where slices meet (partial sums out, ticket, sums back: 7 us
-// measured).
+// measured).  The plan's us is fitted to 3280 calls of one to four layers, r = 0, 8
+// and 64 (6 % rms): the rounds, X read and its planes written, the output, the
+// codes, and for an adapter T1 and its term; where a group's layers are of
+// unequal rows the grid's empty workgroups take slots of full ones (4.5 us once
+// they push it past one round).  The runtime takes the plan where us is below
+// the tiles' estimate plus 1 us (0.2 without an adapter): 2970 of the 3280, 37 of
+// them slower than the tiles by more than 3 %, 7 by more than 6 % (if all were
+// taken 255 and 185: 468 tokens of 136 x 2560 without an adapter 20.7 us against
+// 13.4, 126 of 13904 x 768 60 against 46, 299 of three layers on 576 26 against 17).
 SlimPlan slim_plan(int count, const DevQW *w, const int64_t *r, int64_t M, int x_bf16) {
   SlimPlan p;
   const int cus = slim_cus();
@@ -677,11 +680,19 @@ SlimPlan slim_plan(int count, const DevQW *w, const int64_t *r, int64_t M, int x
     umax = std::max(umax, (w[i].cols + kUnit - 1) / kUnit);
     rmax = std::max(rmax, r[i]);
   }
+  int64_t rows = 0, kmax = 0;
+  double code_mb = 0;
+  for (int i = 0; i < count; ++i) {
+    rows += w[i].rows;
+    kmax = std::max(kmax, w[i].cols);
+    code_mb += (double)((w[i].cols + kUnit - 1) / kUnit) * (double)w[i].rows * 64e-6;
+  }
   const int rhi = p.P * p.G >= 4 && p.G >= 3 ? 3 : 4;  // more spill registers
   double best = 0;
   for (int R = 2; R <= rhi; ++R)
     for (int64_t q = 8; q <= ((umax + 7) / 8) * 8; q += 4) {  // units per workgroup
       int64_t wgs = 0, groups = 0, um = 0;
+      int64_t gx = 0;
       int S[kMaxSlimSegs], smax = 1, nbp = 0;
       for (int i = 0; i < count; ++i) {
         const int64_t U = (w[i].cols + kUnit - 1) / kUnit;
@@ -693,6 +704,7 @@ SlimPlan slim_plan(int count, const DevQW *w, const int64_t *r, int64_t M, int x
         smax = std::max(smax, S[i]);
         wgs += T * S[i] * p.chunks;
         groups += T * p.chunks;
+        gx = std::max(gx, T);
       }
       const uint32_t lds = slim_lds(p.G, R, nbp, rmax);
       if (smax > kMaxSlices || nbp > kMaxNb || groups > kDecodeMaxTiles || lds > kLdsLimit)
@@ -706,6 +718,17 @@ SlimPlan slim_plan(int count, const DevQW *w, const int64_t *r, int64_t M, int x
       p.ok = true;
       p.R = R;
       p.lds = lds;
+      const bool f32 = p.P == 2;
+      const double wu = (double)((um + 7) / 8) * unit / 2400.0, occ = (double)wgs / cus;
+      const double mk = (double)M * (double)kmax * 1e-6;
+      p.us = (f32 ? 3.7 : 3.2) + (double)rounds * (f32 ? 2.5 + 1.13 * wu : 3.2 + 1.06 * wu) +
+             occ * (f32 ? -1.3 : -1.3 + 0.15 * wu) + (smax > 1 ? f32 ? 3.4 : 4.3 : 0.0) +
+             (f32 ? 5.8 : 2.75) * mk + (f32 ? 8.5 : 5.9) * (double)M * (double)rows * 1e-6 +
+             0.175 * code_mb;
+      if (rmax > 0)
+        p.us += (f32 ? 2.3 : 3.0) +
+                (double)((rmax + 15) / 16) * (1.3 * (double)rounds + (f32 ? 0.7 : 1.3) * mk);
+      if (count > 1 && wgs <= cus && gx * smax * p.chunks * count > cus) p.us += 4.5;
       for (int i = 0; i < count; ++i) {
         p.S[i] = S[i];
         p.groups[i] = (int)((w[i].rows + 16 * R - 1) / (16 * R));

@@ -299,6 +299,7 @@ struct SlimPlan {
   bool ok = false;
   int G = 0, P = 0, R = 0, chunks = 0;
   uint32_t lds = 0;
+  double us = 0;  // about what the two launches take
   int S[kMaxSlimSegs] = {}, groups[kMaxSlimSegs] = {}, nz[kMaxSlimSegs] = {};
   size_t part_floats[kMaxSlimSegs] = {};  // scratch of the K slices' sums
   size_t xp_bytes[kMaxSlimSegs] = {};     // scratch of the X planes

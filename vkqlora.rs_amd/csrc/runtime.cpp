@@ -463,23 +463,39 @@ bool takes_slim(const DevQW &W, const qh_lora *l, const void *x, int xdt, int64_
   return qh::slim_ok(W, x, xdt == QH_BF16, l ? l->a : nullptr, M, l ? (int64_t)l->r : 0);
 }
 
+// About what the tile kernels take for T1 (us), fitted with bf16_gemm_us: a rank
+// launch up to K = 2048, else the dense kernel and its reduction.
+double t1_us(int64_t M, int64_t K, int64_t r, bool f32) {
+  if (r == 0) return 0.0;
+  const double k = (double)K * 1e-3, mk = (double)M * (double)K * 1e-6;
+  if (!qh::rank_gemm_ok(K, r)) return (f32 ? 11.3 : 10.6) + k + 1.6 * mk;
+  return (f32 ? 2.9 : 3.2) + k * ((f32 ? 3.55 : 8.5) + 3.6 * (double)((r + 15) / 16 - 1)) + 1.6 * mk;
+}
+double tile_forward_us(const DevQW &W, const qh_lora *l, int xdt, int64_t M) {
+  const bool f32 = xdt != QH_BF16;
+  return qh::bf16_gemm_us(M, W.rows, W.cols, f32, true) + t1_us(M, W.cols, l ? (int64_t)l->r : 0, f32);
+}
+
 // `count` layers, each on its own x (layers with the same x share its
 // preparation); with `beta` y += the result.  False, with nothing launched,
-// where its scratch cannot be had (see Carve::try_bind) or no plan covers the
-// group: the caller runs the layers on the tile kernels.  Their scratch for
+// where its scratch cannot be had (see Carve::try_bind), no plan covers the
+// group, or the tile kernels' `tile_us` is clearly below the plan's (see
+// slim_plan): the caller runs the layers on the tile kernels.  Their scratch for
 // these layers is `tile_bytes`, and the buffer grows to that as well: what
 // this kernel needs does not rise with the token count, so a capture of fewer
 // tokens than the calls before it may find too little for it, but not for
 // the tiles, which then need no more than those calls would have.
 bool slim_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora *const *l,
               const void *const *x, int xdt, int64_t M, float *const *y, float *const *t1_out,
-              int beta, size_t tile_bytes, hipStream_t s) {
+              int beta, size_t tile_bytes, double tile_us, hipStream_t s) {
   if (count > (size_t)qh::kMaxSlimSegs) return false;
   const int xb = xdt == QH_BF16, n = (int)count;
   int64_t rs[qh::kMaxSlimSegs] = {};
   for (int i = 0; i < n; ++i) rs[i] = l[i] ? (int64_t)l[i]->r : 0;
   const qh::SlimPlan pl = qh::slim_plan(n, W, rs, M, xb);
-  if (!pl.ok) return false;
+  bool lora = false;
+  for (int i = 0; i < n; ++i) lora = lora || rs[i] > 0;
+  if (!pl.ok || pl.us > tile_us + (lora ? 1.0 : 0.2)) return false;
   Carve c;
   size_t it[qh::kMaxSlimSegs], ix[qh::kMaxSlimSegs], ip[qh::kMaxSlimSegs];
   int own[qh::kMaxSlimSegs];
@@ -604,7 +620,7 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
   }
   if (takes_slim(W, l, x, xdt, M) &&
       slim_dev(ctx, 1, &W, &l, &x, xdt, M, &y, &t1_out, accumulate ? 1 : 0,
-               TileForward(W, l, x, xe, M, t1_out).c.total(), s))
+               TileForward(W, l, x, xe, M, t1_out).c.total(), tile_forward_us(W, l, xdt, M), s))
     return;
   // Small batches: the MFMA decode kernels (batch <= 16, K % 256 == 0), else
   // the VALU GEMV (batch <= 4, K % 64 == 0); both need 16-byte aligned rows
@@ -1004,14 +1020,20 @@ void forward_shared_dev(qh_ctx *ctx, size_t count, const DevQW *W, const qh_lora
   if (slim) {
     const void *const xs[qh::kMaxSlimSegs] = {x, x, x, x};
     size_t tile_bytes = 0;
+    double tile_us = 0;
+    int64_t rows = 0, r = 0;
     for (size_t i = 0; i < count; ++i) {
       const float *t1i = t1_out ? t1_out[i] : nullptr;
+      rows += W[i].rows, r = std::max(r, l[i] ? (int64_t)l[i]->r : 0);
       if (shared)
         tile_bytes += l[i] && !t1i ? (size_t)M * l[i]->r * 4 + 256 : 0;
       else
-        tile_bytes = std::max(tile_bytes, TileForward(W[i], l[i], x, xe, M, t1i).c.total());
+        tile_bytes = std::max(tile_bytes, TileForward(W[i], l[i], x, xe, M, t1i).c.total()),
+        tile_us += tile_forward_us(W[i], l[i], xdt, M);
     }
-    if (slim_dev(ctx, count, W, l, xs, xdt, M, y, t1_out, 0, tile_bytes, s)) return;
+    if (shared)
+      tile_us = qh::bf16_gemm_us(M, rows, K, xdt != QH_BF16, false) + t1_us(M, K, r, xdt != QH_BF16);
+    if (slim_dev(ctx, count, W, l, xs, xdt, M, y, t1_out, 0, tile_bytes, tile_us, s)) return;
   }
   if (!shared) {
     for (size_t i = 0; i < count; ++i)
