@@ -126,6 +126,27 @@ def test_calls_that_planes_slow_down_stay_off_them(ctx, N, K, M):
         assert "planes" not in fwd and "planes" not in bwd, (fwd, bwd)
 
 
+def test_codes_off_16_bytes_stay_off_planes(ctx):
+    """k_nf4_bf16 reads codes 8 bytes at a time, the planes 16: a weight that
+    starts on 8 bytes stays on the former, with the same bits."""
+    from qlora_hip import device as QD
+    N, K, M = 4096, 1088, 1100
+    L = _layer(QD, ctx, N, K, 8, M, torch.float32, True)
+    W, ys = L["W"], []
+    for off in (0, 8):
+        buf = torch.empty(W.codes.numel() + off, dtype=torch.uint8, device="cuda")
+        buf[off:] = W.codes.reshape(-1)
+        V = QD.DeviceWeight(N, K, 64, buf[off:], scale_codes=W.scale_codes, absmax=W.absmax)
+        ys.append(torch.empty(M, N, device="cuda"))
+        ctx.set_timing(True)
+        QD.forward(V, L["lora"], L["x"], M, ys[-1], ctx=ctx)
+        torch.cuda.synchronize()
+        rep = ctx.timing_report(reset=True)
+        ctx.set_timing(False)
+        assert V.struct().codes % 16 == off and ("planes" in rep) == (off == 0), rep
+    assert torch.equal(ys[0].view(torch.int32), ys[1].view(torch.int32))
+
+
 @pytest.mark.parametrize("Ns,K,M,planes", [
     ((4352, 4352, 4352), 1088, 1024, (False, False)),  # one launch fills its rounds better
     ((2304, 2304, 2304), 2048, 2048, (False, False)),

@@ -172,8 +172,8 @@ __global__ __launch_bounds__(kPlThreads) void k_planes(PlaneJobs A) {
   const int k0 = 256 * kSpan * (b - rt * nk) + 64 * kSpan * wave, r = 32 * rt + l32;
   const int rc = min(r, rows - 1);
   if (q.kind == kNf4Row) {
-    // pieces of 64 k are blocks (K % 64 == 0): a lane pair loads its row's 32
-    // code bytes, lane half h decodes dword 2 t + h for k tile t
+    // pieces of 64 k are blocks (K % 64 == 0, 16-byte aligned codes): a lane pair
+    // loads its row's 32 code bytes, lane half h decodes dword 2 t + h for k tile t
     v4u c0[kSpan], c1[kSpan];
     float s[kSpan];
 #pragma unroll
@@ -533,18 +533,20 @@ double plane_us(int64_t M, int64_t N, int64_t K, bool f32) {
 
 // Planes where their estimate is below that of k_nf4_bf16, in the range measured:
 // more than half a round of 128 x 256 tiles and K of 512 or more, at most 2 GiB of
-// planes (the LoRA term of rank r included).  The pass over the operands costs (8 or 4 bytes) x rows + 4.5 bytes x columns per k,
-// whatever the product, and columns are padded to 256, so that narrow outputs
-// and few rows lose: fp32 20000 x 192 over 2048 188 us against 150, 64 x 128256
-// over 4096 888 against 448, 2048 x 4096 over 512 39 against 37; they win from
-// about 576 columns and 400 rows at K of 1536 (8192 x 576 87 against 97), 1.2
-// times as fast on the geometric mean of the sizes taken here, 1.4 at 1100 x 4096
-// over 4096.  Of 1456 calls measured, fp32 and bf16, forward and input gradient,
-// 719 are taken, 9 of them slower by more than 3 % (at most 7); 125 of the
-// others would be faster by more than 5 % (all of these shapes: 421 slower, up
-// to 3.1 times).  What k_nf4_bf16 splits (at most 128 columns, up to 21760 rows)
-// stays there: its bits are those of the allocation-free backward, which takes
-// no planes.
+// planes (the LoRA term of rank r included).  The pass over the operands costs
+// (8 or 4 bytes) x rows + 4.5 bytes x columns per k, whatever the product, and
+// columns are padded to 256, so that narrow outputs and few rows lose: fp32
+// 20000 x 192 over 2048 188 us against 150, 64 x 128256 over 4096 888 against 448,
+// 2048 x 4096 over 512 39 against 37; they win from about 576 columns and 400 rows
+// at K of 1536 (8192 x 576 87 against 97), 1.2 times as fast on the geometric mean
+// of the sizes taken here, 1.4 at 1100 x 4096 over 4096.  Of 1456 calls measured,
+// fp32 and bf16, forward and input gradient, 719 are taken, 9 of them slower by
+// more than 3 % (at most 7); 125 of the others would be faster by more than 5 %
+// (all of these shapes: 421 slower, up to 3.1 times).  Below 288 rows forwards with
+// an adapter are slower than estimated (223 x 18032 over 4096 in fp32 239 us
+// against 219, 263 x 17416 242 against 229; 300 x 28672 over 8192 624 against 725).
+// What k_nf4_bf16 splits (at most 128 columns, up to 21760 rows) stays there: its
+// bits are those of the allocation-free backward, which takes no planes.
 bool plane_ok(int64_t M, int64_t N, int64_t K, int64_t r, bool f32) {
   return M >= 288 && up(M, 128) * up(N, 256) > 128 && K >= 512 && bf16_gemm_splits(M, N, K) == 1 &&
          M < (1 << 24) && N < (1 << 24) && K < (1 << 24) && r < (1 << 24) &&

@@ -269,8 +269,10 @@ struct PlaneSrc {
   void *dst;
 };
 // Whether an M x N output over K with an adapter of rank r (0: none) and fp32 or
-// bf16 activations goes through planes.
+// bf16 activations goes through planes (PLANE_NF4_ROW: where plane_codes_ok too).
 bool plane_ok(int64_t M, int64_t N, int64_t K, int64_t r, bool f32);
+// Whether the codes can be read as weight rows: 16 bytes at a time.
+inline bool plane_codes_ok(const DevQW &w) { return ((uintptr_t)w.codes & 15) == 0; }
 // About what they then take (us).
 double plane_us(int64_t M, int64_t N, int64_t K, bool f32);
 // Bytes of an A operand's (M rows) and a B operand's (N rows) planes.

@@ -684,7 +684,7 @@ void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
   const bool fast = f.fast, bf16 = f.bf16;
   if (!bf16) writes_y("forward_dev: y += on the fp32 tile engine");
   // large GEMMs through operand planes where their memory can be had
-  bool plane = bf16 && qh::plane_ok(M, N, K, r, xe == qh::E_F32);
+  bool plane = bf16 && qh::plane_codes_ok(W) && qh::plane_ok(M, N, K, r, xe == qh::E_F32);
   Carve cp;
   const PlaneSlots slots(cp, plane, M, N, K, r, xe == qh::E_F32 ? 2 : 1);
   std::vector<char *> pp;
@@ -987,7 +987,8 @@ bool shared_ok(size_t count, const DevQW *W, const qh_lora *const *l, const void
   int64_t sum = 0;
   for (size_t i = 0; i < count && planes; ++i) {
     const int64_t N = W[i].rows, r = l[i] ? (int64_t)l[i]->r : 0;
-    planes = dy ? qh::plane_ok(M, K, N, r, f32) : qh::plane_ok(M, N, K, r, f32);
+    planes = dy ? qh::plane_ok(M, K, N, r, f32)
+                : qh::plane_codes_ok(W[i]) && qh::plane_ok(M, N, K, r, f32);
     us += dy ? qh::plane_us(M, K, N, f32) : qh::plane_us(M, N, K, f32);
     sum += N;
   }
