@@ -244,9 +244,9 @@ def test_empty_reductions(ctx, QD, N, K, M):
 
 @pytest.mark.parametrize("act", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("N,K,M,r", [
-    (4200, 4160, 1100, 16),   # ragged M, N (256 x 128 tiles) and grad_x reduction (4200 rows)
+    (4200, 4160, 1100, 16),   # ragged M, N and grad_x reduction (4200 rows); operand planes
     (4200, 4160, 1100, 0),    # no adapter
-    (4096, 4096, 1024, 64),   # 256 x 256 tiles for grad_x, two LoRA steps
+    (4096, 4096, 1024, 64),   # whole tiles, four k tiles of the LoRA term; operand planes
 ])
 def test_bf16_mfma_path_parity(ctx, QD, N, K, M, r, act):
     """The large GEMMs on bf16 MFMA (weight as hi + lo bf16 parts; bf16

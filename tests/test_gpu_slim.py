@@ -86,6 +86,52 @@ def test_slim_forward(ctx, N, K, r, M, act):
         assert torch.equal(y0.view(torch.int32), L["y"].view(torch.int32))
 
 
+WIDE = [
+    # (N, K, r, M, dtypes): row groups of 48 and 64 rows (three and four 16-row
+    # tiles a wave), each with every count of token groups that has them, rows
+    # past a group; in the comment what slim_plan picks on 256 CUs
+    (8243, 320, 33, 17, "fb"),    # 2 token groups, 3 tiles
+    (12391, 320, 64, 17, "fb"),   # 2, 4
+    (4101, 320, 64, 50, "f"),     # 2, 3 on two workgroups of tokens
+    (6161, 320, 8, 49, "f"),      # 2, 4
+    (2759, 576, 16, 100, "f"),    # 3, 3
+    (4162, 320, 64, 70, "b"),     # 3, 3
+    (6163, 576, 16, 70, "b"),     # 3, 4
+    (4130, 576, 33, 100, "b"),    # 4, 3
+    (9999, 1088, 64, 40, "fb"),   # 3, 3, two rounds
+    (11008, 4096, 16, 37, "fb"),  # a 7B-class MLP's layer
+]
+
+
+@pytest.mark.parametrize("N,K,r,M,acts", WIDE)
+def test_slim_wide_layers(ctx, N, K, r, M, acts):
+    from qlora_hip import device as QD
+    g = torch.Generator(device="cuda").manual_seed(N + K + M)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    w, a, b = rnd(N, K) * 0.02, rnd(r, K) / K ** 0.5, rnd(N, r) * 0.01
+    lora = QD.lora_struct(a, b, r, 16.0)
+    for act in [dict(f=torch.float32, b=torch.bfloat16)[c] for c in acts]:
+        x = rnd(M, K).to(act)
+        xd = x.double()
+        t1w = xd @ a.double().T
+        for dq in (True, False):
+            print(f"slim wide N={N} K={K} r={r} M={M} {act} dq={dq}", flush=True)
+            W = QD.DeviceWeight.quantize(w, 64, dq, ctx=ctx)
+            wd = W.dequantize(ctx=ctx).view(N, K).double()
+            y = torch.full((M, N), float("nan"), device="cuda")
+            t1 = torch.full((M, r), float("nan"), device="cuda")
+            ctx.set_timing(True)
+            QD.forward(W, lora, x, M, y, t1=t1, ctx=ctx)
+            torch.cuda.synchronize()
+            rep = ctx.timing_report(reset=True)
+            ctx.set_timing(False)
+            assert "forward_slim" in rep, rep
+            want = xd @ wd.T + (16.0 / r) * (t1w @ b.double().T)
+            n = lambda t: t.cpu().numpy()  # noqa: E731
+            assert nerr(n(t1), n(t1w), K, n(xd), n(a)) < TOL_T1
+            assert nerr(n(y), n(want), K, n(xd), n(wd)) < TOL[act]
+
+
 def test_slim_shared_layers_of_unequal_rows(ctx):
     """Four layers on one x in one launch: rows of 1 to 11 row groups, one
     without an adapter, K slices in all of them."""
