@@ -97,6 +97,10 @@ QH_API uint32_t qh_abi_version(void);
 /* GpuContext::try_new_blocking (context.rs:33).  QH_NO_DEVICE when no
  * MI355X is visible (*out stays NULL), QH_ERR_GPU on runtime failure. */
 QH_API qh_status qh_ctx_create(qh_ctx **out);
+/* Gives back the device memory that the context's calls grew it to: scratch of
+ * the largest call, and from the first call with large GEMMs on their operand
+ * planes, up to 2 GiB.  Destroy HIP graphs captured on the context first: they
+ * hold addresses in that memory. */
 QH_API void qh_ctx_destroy(qh_ctx *ctx);
 /* Message of the last failing call on this thread ("" if none). */
 QH_API const char *qh_last_error(void);

@@ -741,7 +741,8 @@ hipError_t launch_softmax_ce(const float *logits, const uint32_t *targets, int64
     // 4 float4 per thread in registers, the rest of a longer row streamed:
     // measured 3.6 / 3.5 TB/s at vocab 49152 / 128256 against 2.8 / 3.1 for
     // 12 float4 (the whole 49152 row, 108 VGPRs, one row per CU at a time)
-    // and below for 512- or 256-thread rows: rows overlapping on a CU matter
+    // and below for 512- or 256-thread rows (all with two divisions per value, before
+    // the product with the reciprocal): rows overlapping on a CU matter
     // more than the second read of the streamed part
     if (per <= 4)
       e = QH_CE(4, false);

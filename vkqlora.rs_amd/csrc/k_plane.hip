@@ -10,8 +10,8 @@
 // k_planes splits X (fp32 into hi + lo) and decodes W (hi + lo) once, in the
 // order in which an MFMA operand is read, and k_plane_gemm copies 1 KiB operand
 // tiles straight into LDS (global_load_lds, no registers), so its waves do
-// nothing but LDS reads and MFMAs: MFMA busy 0.73, and the card then runs at
-// 1.84 GHz instead of 2.4 (the product is bound by power: steps of 32 k
+// nothing but LDS reads and MFMAs: MFMA busy 0.72 (fp32; bf16 0.68), and the card then
+// runs at 1.84 GHz instead of 2.4 (the product is bound by power: steps of 32 k
 // with half the barriers ran 13 % more cycles at a 7 % higher clock).  The sums are
 // those of k_nf4_bf16 without a split reduction, in its order: the same bits.
 //
@@ -503,7 +503,9 @@ hipError_t run_plane(const PlaneGemmDev &g0, hipStream_t st) {
 int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Tile rows: the count of rounds of 256 workgroups times a tile's time (its
-// MFMAs, plus a fixed part of a k tile's phases) decides.
+// MFMAs, plus a fixed part of a k tile's phases) decides.  The fixed part is worth
+// 24 rows' MFMAs in fp32 (24.6 fitted to 223 calls of K from 2048 up); with the two
+// MFMAs a product of bf16 the same fit gives 113, and the rule keeps fp32's.
 int plane_bm(int64_t M, int64_t N) {
   int best = 256;
   double bc = 0;

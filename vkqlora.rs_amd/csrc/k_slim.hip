@@ -16,10 +16,14 @@
 // split K, and a wave decodes code bytes straight into MFMA operands through a
 // byte-pair table in LDS, with the next two code loads and the next X tiles
 // in flight.  Block scales multiply a block's partial sum, once per output.
-// Per 128 of K and 48 fp32 tokens a wave spends about 1150 cycles per 16 rows
-// on the matrix cores and 3100 on its X tiles (64 bytes a cycle from L2,
-// whatever R is), so R is as large as the registers allow where that leaves
-// one workgroup per CU.  More tokens take workgroups of their own (the codes
+// Per 128 of K and 48 fp32 tokens the two waves of a SIMD need 1150 cycles per 16
+// rows on the matrix cores (36 MFMAs of 16 cycles each) and the CU's eight waves
+// 192 KiB of X tiles, 3100 cycles at 64 bytes a cycle from L2, whatever R is, so
+// R is as large as the registers allow where that leaves one workgroup per CU.
+// The kernel comes to less than half of either: at 37 fp32 tokens 16.3 us for
+// 4096 x 4096, 22.4 for 11008 x 4096 (MFMA busy 0.19), 26.4 for 4096 x 11008, of which
+// 7.1 to 7.5 are a workgroup's start and end (all of a K of 384), after 6.4 to 8 us of
+// preparation.  More tokens take workgroups of their own (the codes
 // come from L2 again); K is split over workgroups only where rows are few
 // (the last one of a group adds the slices in order).
 //
@@ -205,7 +209,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_slim(SlimArgs A, uint32_t o_fla
     }
   }
 
-  // ---- the slice's block scales into LDS: [16 R rows][nbp], exact fp32.
+  // ---- the slice's block scales into LDS: [16 R rows][nbp], the exact fp32 scale
+  // times the rounded 1 / kAlpha (one more rounding).
   // TPR threads a row, blocks j, j + TPR, ... of it each.
   const int nb = 2 * nu_s, kb0 = 2 * us0, nbp = L.nbp;
   constexpr uint32_t o_sc = kTabBytes;
@@ -649,7 +654,7 @@ bool slim_ok(const DevQW &w, const void *x, int x_bf16, const float *a, int64_t 
 // Token groups: as many as fit (48 fp32 or 64 bf16 tokens a workgroup), evenly
 // over the workgroups that share them.  (R, units of K per workgroup): the
 // cheapest estimate in cycles of a CU, rounds of one workgroup per CU times
-//  * 18000 for a workgroup's start and end (about 8 us measured: arguments,
+//  * 18000 for a workgroup's start and end (7.1 to 7.5 us measured: arguments,
 //    first loads, table, last sum),
 //  * per unit of a wave (two waves per SIMD) the larger of its code bytes at
 //    the CU's share of HBM and its MFMAs plus its X tiles at 64 bytes a cycle

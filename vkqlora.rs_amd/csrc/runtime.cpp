@@ -445,8 +445,9 @@ bool takes_split(const DevQW &W, const qh_lora *l, const void *x, int64_t M) {
 }
 
 // True when forward_dev with `accumulate` can add its result to y in the
-// GEMM (the bf16-MFMA path: its epilogue, or its split-K reduction);
-// otherwise a caller that wants y += forward(x) computes into a buffer and
+// GEMM (the few-token kernel, operand planes and k_nf4_bf16, by their epilogue or
+// the reduction of their split sums: what is true here may take any of the
+// three); otherwise a caller that wants y += forward(x) computes into a buffer and
 // adds.
 static bool forward_accumulates(const DevQW &W, const qh_lora *l, const void *x, size_t batch) {
   const int64_t M = (int64_t)batch, N = W.rows, K = W.cols;
@@ -593,9 +594,9 @@ struct TileForward {
 };
 
 // ---- fused forward on device pointers -----------------------------------
-// With `accumulate` y += the result; only the bf16-MFMA path (the one
-// forward_accumulates names) does that, every other path refuses it before
-// launching anything (forward_add_dev picks).
+// With `accumulate` y += the result; only the paths that forward_accumulates names
+// do that, every other path refuses it before launching anything
+// (forward_add_dev picks).
 void forward_dev(qh_ctx *ctx, const DevQW &W, const qh_lora *l, const void *x,
                  int xdt, size_t batch, float *y, float *t1_out, hipStream_t s,
                  bool accumulate = false) {
