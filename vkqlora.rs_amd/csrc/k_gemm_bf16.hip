@@ -1048,8 +1048,8 @@ bool bf16_gemm_ok(const DevQW &w, const void *a, int64_t lda, int64_t K) {
 
 int bf16_gemm_splits(int64_t M, int64_t N, int64_t K) { return plan_for(M, N, K).splits; }
 
-// Fitted to some 1500 forwards and input gradients (16 to 65536 rows and columns,
-// K 320 to 11008): within 6 % rms, 4 % above 40 us.  A step of 32 k costs what the
+// Fitted to some 2000 forwards and input gradients (16 to 65536 rows and columns, K
+// 320 to 11008): within 6 % rms, 3 % above 40 us.  A step of 32 k costs what the
 // rounds of workgroups take at full and at partial occupancy (two blocks of the
 // medium tier fit a CU where it has more tiles than CUs, four small ones do),
 // plus the tiles' share of operand traffic.
@@ -1057,13 +1057,16 @@ double bf16_gemm_us(int64_t M, int64_t N, int64_t K, bool f32, bool split) {
   const Plan p = plan_for(M, N, K);
   const auto up = [](int64_t a, int64_t b) { return (double)((a + b - 1) / b); };
   const int64_t steps = (K + kBK - 1) / kBK;
-  const double mn = (double)M * (double)N * 1e-6;
+  const double mn = (double)M * (double)N * 1e-6, mk = (double)M * (double)K * 1e-6;
   if (p.tier == kLarge) {
     const bool wide = wide_tiles(M, N);
-    const double t = up(M, 256) * up(N, wide ? 256 : 128), R = up((int64_t)t, 256);
-    const double step = wide ? f32 ? 1.49 * R + 0.0042 * t : 1.15 * R + 0.0026 * t
-                             : f32 ? 1.28 * R + 0.0011 * t : 0.96 * R + 0.00055 * t;
-    return (wide ? 3.5 + 2 * R : 9 + R) + (double)steps * step + (f32 ? 0.45 : 0.35) * mn;
+    const double t = up(M, 256) * up(N, wide ? 256 : 128), wg = t / 256, R = up((int64_t)t, 256);
+    const double s = (double)steps;
+    if (wide)
+      return f32 ? 0.5 + s * (1.383 * R + 1.204 * wg) + 1.7 * R + 0.55 * mn + 0.19 * mk
+                 : 1.8 + s * (1.083 * R + 0.732 * wg) + 4.6 * R + 0.395 * mn + 0.04 * mk;
+    return f32 ? 5.3 + s * (1.16 * R + 0.368 * wg) + 3.5 * R + 0.185 * mn + 0.525 * mk
+               : 5.4 + s * (0.866 * R + 0.2 * wg) + 6.3 * R - 0.15 * mn + 0.3 * mk;
   }
   const int sp = split ? p.splits : 1;
   const double tile = p.tier == kMedium ? 128 : 64, t = up(M, (int64_t)tile) * up(N, (int64_t)tile);
@@ -1075,7 +1078,8 @@ double bf16_gemm_us(int64_t M, int64_t N, int64_t K, bool f32, bool split) {
     return 5.6 + ks * (f32 ? 0.95 + 0.9 * (R - 1) + 0.09 * wg : 0.8 + 0.72 * (R - 1)) +
            (sp > 1 ? 0.18 + 2.85 * sp * mn : 0) + (f32 ? 0.7 : 0.5) * mn;
   const double R2 = up((int64_t)t * sp, 512);
-  return 6.9 + ks * (0.295 * R2 + (f32 ? 0.43 * R + 0.3175 * wg : 0.33 * R + 0.16 * wg)) + 0.23 * mn;
+  return f32 ? 5.8 + ks * (0.277 * R2 + 0.467 * R + 0.285 * wg) + 0.36 * mn + 0.15 * mk
+             : 6.2 + ks * (0.258 * R2 + 0.393 * R + 0.126 * wg) + 0.3 * mn + 0.044 * mk;
 }
 
 hipError_t launch_gemm_bf16(const Bf16GemmArgs &g, int w_form, int a_f32, int splits,

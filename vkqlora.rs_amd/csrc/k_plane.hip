@@ -503,14 +503,15 @@ hipError_t run_plane(const PlaneGemmDev &g0, hipStream_t st) {
 int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Tile rows: the count of rounds of 256 workgroups times a tile's time (its
-// MFMAs, plus a fixed part of a k tile's phases) decides.  The fixed part is worth
-// 24 rows' MFMAs in fp32 (24.6 fitted to 223 calls of K from 2048 up); with the two
-// MFMAs a product of bf16 the same fit gives 113, and the rule keeps fp32's.
+// MFMAs, plus a fixed part of a k tile's phases worth those of 80 rows) decides.
+// Measured over 637 calls on which constants from 12 to 112 disagree: 64 to 112 come
+// within 0.2 % of the best height on the mean (fp32 at most 3 %, bf16 11), 24 loses 4.7 %
+// in fp32 (up to 24) and 12 % in bf16 (up to 38).
 int plane_bm(int64_t M, int64_t N) {
   int best = 256;
   double bc = 0;
   for (int bm : {256, 192, 128}) {
-    const double c = (double)up(up(M, bm) * up(N, 256), 256) * (bm + 24);
+    const double c = (double)up(up(M, bm) * up(N, 256), 256) * (bm + 80);
     if (bc == 0 || c < bc) bc = c, best = bm;
   }
   return best;
@@ -518,19 +519,22 @@ int plane_bm(int64_t M, int64_t N) {
 
 }  // namespace
 
-// About what the planes and the GEMM take (us): their bytes, the rounds of
+// About what the planes and the GEMM take (us): the planes' bytes (dearer past the
+// 200 MB that stay in the last-level cache until the GEMM reads them), the rounds of
 // tiles, the tiles' operand traffic and the output.  Fitted to the same calls as
-// bf16_gemm_us, 5 to 6 % rms; the constant is 3 us above the fit, for the calls
-// below 40 us.
+// bf16_gemm_us, 4 % rms; the constant is 1 us above the fit, for the calls below 40
+// us.
 double plane_us(int64_t M, int64_t N, int64_t K, bool f32) {
   const int bm = plane_bm(M, N);
-  const double m = (double)M, n = (double)N, k = (double)K;
+  const double mk = (double)M * (double)K * 1e-6, nk = (double)N * (double)K * 1e-6;
+  const double mn = (double)M * (double)N * 1e-6, k = (double)K * 1e-3;
   const double t = (double)(up(M, bm) * up(N, 256)), R = (double)up((int64_t)t, 256);
+  const double over = std::max(0.0, (f32 ? 4 : 2) * mk + 4 * nk - 200);
   if (f32)
-    return 13 + (1.36 * m + 0.97 * n) * k * 1e-6 + k * (R * (bm + 24) * 107e-6 + t * bm * 54e-8) +
-           m * n * 0.48e-6 + R * bm * 0.0135;
-  return 15.7 + (0.62 * m + 1.03 * n) * k * 1e-6 + k * (R * (bm + 24) * 105e-6 + t * bm * 19.5e-8) +
-         m * n * 1.05e-6 - R * bm * 0.021;
+    return 7.2 + 1.18 * mk + 0.82 * nk + 0.134 * over +
+           k * (R * (0.82 + 0.0978 * bm) + 0.000662 * t * bm) + 10.4 * R;
+  return 9.5 + 0.49 * mk + 0.83 * nk + 0.164 * over +
+         k * (R * (7.34 + 0.044 * bm) + 0.000397 * t * bm) + 0.286 * mn + 6.6 * R;
 }
 
 // Planes where their estimate is below that of k_nf4_bf16, in the range measured:
@@ -541,12 +545,12 @@ double plane_us(int64_t M, int64_t N, int64_t K, bool f32) {
 // 20000 x 192 over 2048 188 us against 150, 64 x 128256 over 4096 888 against 448,
 // 2048 x 4096 over 512 39 against 37; they win from about 576 columns and 400 rows
 // at K of 1536 (8192 x 576 87 against 97), 1.2 times as fast on the geometric mean
-// of the sizes taken here, 1.4 at 1100 x 4096 over 4096.  Of 1456 calls measured,
-// fp32 and bf16, forward and input gradient, 719 are taken, 9 of them slower by
-// more than 3 % (at most 7); 125 of the others would be faster by more than 5 %
-// (all of these shapes: 421 slower, up to 3.1 times).  Below 288 rows forwards with
-// an adapter are slower than estimated (223 x 18032 over 4096 in fp32 239 us
-// against 219, 263 x 17416 242 against 229; 300 x 28672 over 8192 624 against 725).
+// of the sizes taken here, 1.4 at 1100 x 4096 over 4096.  Of 2347 calls measured,
+// fp32 and bf16, forward and input gradient, 1805 are taken, 32 of them slower by
+// more than 3 % (14 by more than 6, at most 20); 32 of the others would be faster by
+// more than 5 % (if all were taken 397 slower, up to 2.3 times).  Below 288 rows
+// forwards with an adapter are slower than estimated (223 x 18032 over 4096 in fp32
+// 239 us against 219, 263 x 17416 242 against 229).
 // What k_nf4_bf16 splits (at most 128 columns, up to 21760 rows) stays there: its
 // bits are those of the allocation-free backward, which takes no planes.
 bool plane_ok(int64_t M, int64_t N, int64_t K, int64_t r, bool f32) {
@@ -555,7 +559,7 @@ bool plane_ok(int64_t M, int64_t N, int64_t K, int64_t r, bool f32) {
          plane_a_bytes(M, K, 2) + plane_b_bytes(N, K) + plane_a_bytes(M, r, 2) +
                  plane_b_bytes(N, r) <=
              (size_t)2 << 30 &&
-         plane_us(M, N, K, f32) < 0.98 * bf16_gemm_us(M, N, K, f32, true);
+         plane_us(M, N, K, f32) < bf16_gemm_us(M, N, K, f32, true);
 }
 
 size_t plane_a_bytes(int64_t M, int64_t K, int parts) {
