@@ -502,16 +502,19 @@ hipError_t run_plane(const PlaneGemmDev &g0, hipStream_t st) {
 
 int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Tile rows: the count of rounds of 256 workgroups times a tile's time (its
-// MFMAs, plus a fixed part of a k tile's phases worth those of 80 rows) decides.
-// Measured over 637 calls on which constants from 12 to 112 disagree: 64 to 112 come
-// within 0.2 % of the best height on the mean (fp32 at most 3 %, bf16 11), 24 loses 4.7 %
-// in fp32 (up to 24) and 12 % in bf16 (up to 38).
-int plane_bm(int64_t M, int64_t N) {
+// Tile rows: the count of rounds of 256 workgroups times a tile's time decides: its
+// MFMAs plus a fixed part, in fp32 a round's start and end (those of 120000 rows
+// over one k: 12 us), in bf16 mostly a k tile's phases (of 80 rows).  Measured over
+// 636 calls whose height depends on the fixed part (taken as 12 to 112 rows): within
+// 0.2 % of the best height on the mean, at most 4 % in fp32 and 12 in bf16; 24 rows lose
+// 5 % in fp32 (up to 24) and 12.5 in bf16 (up to 38), 80 rows 2 % of a 70B-class block in
+// fp32, whose long reductions hide a round's ends.
+int plane_bm(int64_t M, int64_t N, int64_t K, bool f32) {
+  const double fixed = f32 ? 120000.0 / (double)K : 80.0;
   int best = 256;
   double bc = 0;
   for (int bm : {256, 192, 128}) {
-    const double c = (double)up(up(M, bm) * up(N, 256), 256) * (bm + 80);
+    const double c = (double)up(up(M, bm) * up(N, 256), 256) * (bm + fixed);
     if (bc == 0 || c < bc) bc = c, best = bm;
   }
   return best;
@@ -521,23 +524,25 @@ int plane_bm(int64_t M, int64_t N) {
 
 // About what the planes and the GEMM take (us): the planes' bytes (dearer past the
 // 200 MB that stay in the last-level cache until the GEMM reads them), the rounds of
-// tiles, the tiles' operand traffic and the output.  Fitted to the same calls as
-// bf16_gemm_us, 4 % rms; the constant is 1 us above the fit, for the calls below 40
-// us.
+// tiles, the tiles' operand traffic (less of it where each XCD has its run of tiles)
+// and the output.  Fitted to 3000 calls of up to 4e12 products, 3.6 % rms in fp32 and 4.7
+// in bf16; the constant is 2 us above the fit, for the calls below 40 us.
 double plane_us(int64_t M, int64_t N, int64_t K, bool f32) {
-  const int bm = plane_bm(M, N);
+  const int bm = plane_bm(M, N, K, f32);
   const double mk = (double)M * (double)K * 1e-6, nk = (double)N * (double)K * 1e-6;
   const double mn = (double)M * (double)N * 1e-6, k = (double)K * 1e-3;
-  const double t = (double)(up(M, bm) * up(N, 256)), R = (double)up((int64_t)t, 256);
+  const int64_t tiles = up(M, bm) * up(N, 256);
+  const double R = (double)up(tiles, 256), rows = (double)tiles * bm * 1e-3;
   const double over = std::max(0.0, (f32 ? 4 : 2) * mk + 4 * nk - 200);
+  const bool xcd = tiles % 8 == 0;
   if (f32)
-    return 7.2 + 1.18 * mk + 0.82 * nk + 0.134 * over +
-           k * (R * (0.82 + 0.0978 * bm) + 0.000662 * t * bm) + 10.4 * R;
-  return 9.5 + 0.49 * mk + 0.83 * nk + 0.164 * over +
-         k * (R * (7.34 + 0.044 * bm) + 0.000397 * t * bm) + 0.286 * mn + 6.6 * R;
+    return 9.2 + 1.09 * mk + 0.81 * nk + 0.123 * over +
+           k * (R * (2.5 + 0.0975 * bm) + (xcd ? 0.619 : 0.666) * rows) + 0.16 * mn + 7.9 * R;
+  return 9.3 + 0.38 * mk + 0.845 * nk + 0.145 * over +
+         k * (R * (8 + 0.0394 * bm) + (xcd ? 0.403 : 0.459) * rows) + 0.255 * mn + 7.7 * R;
 }
 
-// Planes where their estimate is below that of k_nf4_bf16, in the range measured:
+// Planes where their estimate is not 3 % above that of k_nf4_bf16, in the range measured:
 // more than half a round of 128 x 256 tiles and K of 512 or more, at most 2 GiB of
 // planes (the LoRA term of rank r included).  The pass over the operands costs
 // (8 or 4 bytes) x rows + 4.5 bytes x columns per k, whatever the product, and
@@ -545,10 +550,10 @@ double plane_us(int64_t M, int64_t N, int64_t K, bool f32) {
 // 20000 x 192 over 2048 188 us against 150, 64 x 128256 over 4096 888 against 448,
 // 2048 x 4096 over 512 39 against 37; they win from about 576 columns and 400 rows
 // at K of 1536 (8192 x 576 87 against 97), 1.2 times as fast on the geometric mean
-// of the sizes taken here, 1.4 at 1100 x 4096 over 4096.  Of 2347 calls measured,
-// fp32 and bf16, forward and input gradient, 1805 are taken, 32 of them slower by
-// more than 3 % (14 by more than 6, at most 20); 32 of the others would be faster by
-// more than 5 % (if all were taken 397 slower, up to 2.3 times).  Below 288 rows
+// of the sizes taken here, 1.4 at 1100 x 4096 over 4096.  Of 2572 calls measured,
+// fp32 and bf16, forward and input gradient, 2055 are taken, 36 of them slower by
+// more than 3 % (17 by more than 6, at most 21); 23 of the others would be faster by
+// more than 5 % (if all were taken 402 slower, up to 2.3 times).  Below 288 rows
 // forwards with an adapter are slower than estimated (223 x 18032 over 4096 in fp32
 // 239 us against 219, 263 x 17416 242 against 229).
 // What k_nf4_bf16 splits (at most 128 columns, up to 21760 rows) stays there: its
@@ -559,7 +564,7 @@ bool plane_ok(int64_t M, int64_t N, int64_t K, int64_t r, bool f32) {
          plane_a_bytes(M, K, 2) + plane_b_bytes(N, K) + plane_a_bytes(M, r, 2) +
                  plane_b_bytes(N, r) <=
              (size_t)2 << 30 &&
-         plane_us(M, N, K, f32) < bf16_gemm_us(M, N, K, f32, true);
+         plane_us(M, N, K, f32) < 1.03 * bf16_gemm_us(M, N, K, f32, true);
 }
 
 size_t plane_a_bytes(int64_t M, int64_t K, int parts) {
@@ -606,7 +611,7 @@ hipError_t launch_plane_gemm(const PlaneGemm &p, hipStream_t st) {
   g.KT = (int)up(p.K, 16);
   g.KT2 = (int)up(p.K2, 16);
   g.beta = p.beta;
-  const int bm = plane_bm(p.M, p.N);
+  const int bm = plane_bm(p.M, p.N, p.K, p.a_parts == 2);
   if (p.a_parts == 2) {
     if (bm == 256) return run_plane<Pl<256, 2>>(g, st);
     if (bm == 192) return run_plane<Pl<192, 2>>(g, st);

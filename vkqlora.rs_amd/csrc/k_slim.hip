@@ -666,8 +666,8 @@ bool slim_ok(const DevQW &w, const void *x, int x_bf16, const float *a, int64_t 
 // codes, and for an adapter T1 and its term; where a group's layers are of
 // unequal rows the grid's empty workgroups take slots of full ones (4.5 us once
 // they push it past one round).  The runtime takes the plan where us is below
-// the tiles' estimate plus 1 us (0.2 without an adapter): 2970 of the 3280, 37 of
-// them slower than the tiles by more than 3 %, 7 by more than 6 % (if all were
+// the tiles' estimate plus 1 us (0.2 without an adapter): 2979 of the 3280, 40 of
+// them slower than the tiles by more than 3 %, 8 by more than 6 % (if all were
 // taken 255 and 185: 468 tokens of 136 x 2560 without an adapter 20.7 us against
 // 13.4, 126 of 13904 x 768 60 against 46, 299 of three layers on 576 26 against 17).
 SlimPlan slim_plan(int count, const DevQW *w, const int64_t *r, int64_t M, int x_bf16) {
